@@ -164,6 +164,7 @@ extern "C" int exa_init(int device) {
   EXA_CHECK(exa_pred_init_5(host, hostf));
   EXA_CHECK(exa_pred_init_6(host, hostf));
   EXA_CHECK(exa_pred_init_7(host, hostf));
+  EXA_CHECK(exa_pred_history_init(host, hostf));
   EXA_CHECK(exa_pred_staged_init(host, hostf));
   EXA_CHECK(exa_pde_init(host));
   if (exa_pde_user_init_all(host) != 0) {
@@ -273,6 +274,19 @@ static bool predictor_staged(const exa_aderdg_config& c, int dev) {
   if (c.order >= 8 || c.contraction == EXA_CONTRACT_STAGED) return true;
   return c.order == 7 && c.precision == EXA_PREC_FP64 && c.contraction == EXA_CONTRACT_DEFAULT &&
          g_tuned[dev & 63][7][EXA_PREC_FP64].contraction == 0;  // exa_autotune's choice wins
+}
+
+// The default predictor of the Euler equations in FP64 or with FP32 sweeps
+// (pred_history.hip; faster than every other form at orders 4..8, see
+// aderdg_history.h), unless the configuration or exa_autotune asks for another
+// form.  Below, cells are too small for it to matter (N = 3, 45^3 cells: 1.16
+// against 1.25 ms FP64, 1.37 against 1.14 mixed); at order 9 its registers do not hold
+// the state (7.8 ms against the staged form's 6.8 at 18^3 cells, FP64).
+static bool predictor_history(const exa_aderdg_config& c, int dev) {
+  return c.pde == EXA_PDE_EULER && !c.linear && c.order >= EXA_HISTORY_MIN_ORDER &&
+         c.order <= EXA_HISTORY_MAX_ORDER &&
+         (c.precision == EXA_PREC_FP64 || c.precision == EXA_PREC_FP32) && c.contraction == EXA_CONTRACT_DEFAULT &&
+         c.waves_per_simd == 0 && g_tuned[dev & 63][c.order][c.precision].contraction == 0;
 }
 
 // Launch extras of a single-grid predictor launch: the gravity source of
@@ -949,7 +963,14 @@ static int batch_run_predictions(exa_solver* s) {
   nodbg.lQi = nodbg.lFi = nodbg.lQhi = nodbg.lFhi = nullptr;
   EXA_ORDER_SWITCH(N, {
     using O = exa::Ord<NN>;
-    if (predictor_staged(s->cfg, s->device)) {
+    if (predictor_history(s->cfg, s->device)) {
+      hipLaunchKernelGGL(exa_pred_history_kernel(NN, s->cfg.precision == EXA_PREC_FP32, s->cfg.fp64_sweeps),
+                         dim3((unsigned)n), dim3(O::NT),
+                         (size_t)exa_pred_history_lds_bytes(NN, s->cfg.precision == EXA_PREC_FP32, s->cfg.fp64_sweeps),
+                         s->stream, s->b_luh.as<double>(),
+                         s->b_lduh.as<double>(), s->b_qf.as<double>(), s->b_ff.as<double>(), s->b_iters.as<int>(),
+                         nullptr, 0.0, 0.0, 0.0, s->cfg.gamma, s->cfg.fp64_sweeps, nullptr, nodbg, ens);
+    } else if (predictor_staged(s->cfg, s->device)) {
       int slots = 0;
       EXA_TRY(staged_slots(NN, s->device, n, &slots));
       EXA_TRY(s->b_stage.ensure(staged_slot_bytes(NN) * (size_t)slots));
@@ -1170,7 +1191,7 @@ extern "C" int exa_grid_create(exa_solver* s, int nx, int ny, int nz, const doub
     delete g;
     return r;
   }
-  g->staged = predictor_staged(s->cfg, s->device);
+  g->staged = predictor_staged(s->cfg, s->device) && !predictor_history(s->cfg, s->device);
   if (g->staged) {
     if ((r = staged_slots(s->cfg.order, s->device, g->nc, &g->nslots)) != EXA_OK ||
         (r = g->stage.ensure(staged_slot_bytes(s->cfg.order) * (size_t)g->nslots)) != EXA_OK) {
@@ -1420,6 +1441,14 @@ int exa_solver_predictor(const exa_solver* s, PredFn* fn, int* threads, size_t* 
   EXA_ARG(N >= 1 && N <= 7, "orders 1..7 (the register-form predictor)");
   EXA_ORDER_SWITCH(N, {
     using O = exa::Ord<NN>;
+    // the FP32 variant's uniform cells take the FP64 predictor's steps bit for
+    // bit: both have to come from the same family of kernels
+    if (predictor_history(s->cfg, s->device) && g_tuned[s->device & 63][NN][EXA_PREC_FP64].contraction == 0) {
+      *fn = exa_pred_history_kernel(NN, s->cfg.precision == EXA_PREC_FP32, s->cfg.fp64_sweeps, true);
+      *threads = O::NT;
+      *lds = exa_pred_history_lds_bytes(NN, s->cfg.precision == EXA_PREC_FP32, s->cfg.fp64_sweeps, true);
+      return EXA_OK;
+    }
     const int wpe = predictor_waves_per_simd(s->cfg, NN, s->device);
     const int form = predictor_form(s->cfg, NN, s->device);
     // the adaptive mesh is mostly uniform away from its features: FP32
@@ -1499,7 +1528,15 @@ static int enqueue_step(exa_grid* g, bool timed) {
     using O = exa::Ord<NN>;
     exa::Ens ex = launch_extras(g->s->cfg);
     ex.fold_update = 1;  // k_riemann_update follows
-    if (g->staged) {
+    if (predictor_history(g->s->cfg, g->s->device)) {
+      hipLaunchKernelGGL(exa_pred_history_kernel(NN, g->s->cfg.precision == EXA_PREC_FP32, g->s->cfg.fp64_sweeps),
+                         dim3((unsigned)g->nc), dim3(O::NT),
+                         (size_t)exa_pred_history_lds_bytes(NN, g->s->cfg.precision == EXA_PREC_FP32, g->s->cfg.fp64_sweeps),
+                         g->stream, g->luh.as<double>(),
+                         g->lduh.as<double>(), g->qf.as<double>(), g->ff.as<double>(), g->iters.as<int>(),
+                         g->dt_cur(), g->dx[0], g->dx[1], g->dx[2], g->s->cfg.gamma, g->s->cfg.fp64_sweeps,
+                         g->iter_sum(), nodbg, ex);
+    } else if (g->staged) {
       hipLaunchKernelGGL(exa_pred_staged_kernel(NN, false, g->s->cfg.pde == EXA_PDE_EULER_GRAVITY,
                                                 g->s->cfg.precision == EXA_PREC_FP32),
                          dim3((unsigned)g->nslots), dim3(O::NT),
@@ -1909,10 +1946,13 @@ static int enqueue_ensemble_step(exa_ensemble* e) {
     const exa_aderdg_config& cfg = gr->s->cfg;
     EXA_ORDER_SWITCH(gr->order, {
       using O = exa::Ord<NN>;
-      const int wpe = predictor_waves_per_simd(cfg, NN, gr->s->device);
-      const int form = predictor_form(cfg, NN, gr->s->device);
-      PredFn kern = predictor_kernel<NN>(false, cfg.precision, wpe, form);
-      hipLaunchKernelGGL(kern, dim3((unsigned)gr->nc), dim3(O::NT), O::LDS_DOUBLES * sizeof(double), e->stream,
+      const bool hist = predictor_history(cfg, gr->s->device);
+      PredFn kern = hist ? exa_pred_history_kernel(NN, cfg.precision == EXA_PREC_FP32, cfg.fp64_sweeps)
+                         : predictor_kernel<NN>(false, cfg.precision, predictor_waves_per_simd(cfg, NN, gr->s->device),
+                                                predictor_form(cfg, NN, gr->s->device));
+      const size_t lds = hist ? exa_pred_history_lds_bytes(NN, cfg.precision == EXA_PREC_FP32, cfg.fp64_sweeps)
+                              : O::LDS_DOUBLES * sizeof(double);
+      hipLaunchKernelGGL(kern, dim3((unsigned)gr->nc), dim3(O::NT), lds, e->stream,
                          gr->luh.as<double>(), gr->lduh.as<double>(), gr->qf.as<double>(), gr->ff.as<double>(),
                          gr->iters.as<int>(), nullptr, 1.0, 1.0, 1.0, 1.4, cfg.fp64_sweeps,
                          gr->iter_sum.as<unsigned long long>(), nodbg, en);
@@ -2028,40 +2068,45 @@ extern "C" int exa_autotune(int order, int precision, int ncells, int* waves_per
   ic.eps = 5.0;
   ic.uinf[0] = ic.uinf[1] = 1.0;
   ic.rho_inf = ic.p_inf = 1.0;
-  double best = 1e300;
+  // average predictor time (ms) of one variant; 0, 0: the default
+  auto variant = [&](int w, int cform, double* t) -> int {
+    exa_aderdg_config cfg{};
+    cfg.order = order;
+    cfg.nvar = 5;
+    cfg.cfl = 0.9;
+    cfg.gamma = 1.4;
+    cfg.pde = EXA_PDE_EULER;
+    cfg.precision = precision;
+    cfg.fp64_sweeps = 1;
+    cfg.waves_per_simd = w;
+    cfg.contraction = cform;
+    exa_solver* s = nullptr;
+    exa_grid* g = nullptr;
+    EXA_TRY(exa_aderdg_create(&cfg, &s));
+    int r = exa_grid_create(s, ncells, ncells, ncells, nullptr, nullptr, &g);
+    *t = 1e300;
+    if (r == EXA_OK) r = exa_grid_set_initial_conditions(g, &ic);
+    if (r == EXA_OK) r = exa_grid_compute_dt(g, nullptr);
+    if (r == EXA_OK) r = exa_grid_step(g, 1);
+    if (r == EXA_OK) r = exa_grid_enable_timing(g, 1);
+    if (r == EXA_OK) {
+      double tt[3];
+      long long cc[3];
+      r = exa_grid_kernel_times(g, tt, cc);
+      if (r == EXA_OK) r = exa_grid_step(g, 3);
+      if (r == EXA_OK) r = exa_grid_kernel_times(g, tt, cc);
+      if (r == EXA_OK && cc[0] > 0) *t = tt[0] / cc[0];
+    }
+    exa_grid_destroy(g);
+    exa_aderdg_destroy(s);
+    return r;
+  };
+  double best = 1e300, deflt = 1e300;
   int bw = 0, bc = 0, k = 0;
   for (int w = 1; w <= 2; ++w)
     for (int cform = EXA_CONTRACT_PENCIL; cform <= EXA_CONTRACT_PENCIL_PAIR; ++cform, ++k) {
-      exa_aderdg_config cfg{};
-      cfg.order = order;
-      cfg.nvar = 5;
-      cfg.cfl = 0.9;
-      cfg.gamma = 1.4;
-      cfg.pde = EXA_PDE_EULER;
-      cfg.precision = precision;
-      cfg.fp64_sweeps = 1;
-      cfg.waves_per_simd = w;
-      cfg.contraction = cform;
-      exa_solver* s = nullptr;
-      exa_grid* g = nullptr;
-      EXA_TRY(exa_aderdg_create(&cfg, &s));
-      int r = exa_grid_create(s, ncells, ncells, ncells, nullptr, nullptr, &g);
       double t = 1e300;
-      if (r == EXA_OK) r = exa_grid_set_initial_conditions(g, &ic);
-      if (r == EXA_OK) r = exa_grid_compute_dt(g, nullptr);
-      if (r == EXA_OK) r = exa_grid_step(g, 1);
-      if (r == EXA_OK) r = exa_grid_enable_timing(g, 1);
-      if (r == EXA_OK) {
-        double tt[3];
-        long long cc[3];
-        r = exa_grid_kernel_times(g, tt, cc);
-        if (r == EXA_OK) r = exa_grid_step(g, 3);
-        if (r == EXA_OK) r = exa_grid_kernel_times(g, tt, cc);
-        if (r == EXA_OK && cc[0] > 0) t = tt[0] / cc[0];
-      }
-      exa_grid_destroy(g);
-      exa_aderdg_destroy(s);
-      if (r != EXA_OK) return r;
+      EXA_TRY(variant(w, cform, &t));
       if (ms) ms[k] = t;
       if (t < best) {
         best = t;
@@ -2069,8 +2114,14 @@ extern "C" int exa_autotune(int order, int precision, int ncells, int* waves_per
         bc = cform;
       }
     }
-  g_tuned[dev & 63][order][precision].wpe = bw;
-  g_tuned[dev & 63][order][precision].contraction = bc;
+  // solvers left at the defaults take the fastest of the six unless the
+  // untuned default is faster still
+  g_tuned[dev & 63][order][precision] = TunedVariant{};
+  EXA_TRY(variant(0, EXA_CONTRACT_DEFAULT, &deflt));
+  if (best < deflt) {
+    g_tuned[dev & 63][order][precision].wpe = bw;
+    g_tuned[dev & 63][order][precision].contraction = bc;
+  }
   if (waves_per_simd) *waves_per_simd = bw;
   if (contraction) *contraction = bc;
   return EXA_OK;
