@@ -565,7 +565,7 @@ k_predictor_history(const double* __restrict__ luh, double* __restrict__ lduh, d
   }
   if (n.s == 0) {
     if (iters) iters[cell] = it;
-    if (sweep_count) atomicAdd(sweep_count, (unsigned long long)it);
+    count_sweeps(sweep_count, cell, it);
   }
 }
 

@@ -918,7 +918,7 @@ __global__ __launch_bounds__(Ord<N>::NT) __attribute__((amdgpu_waves_per_eu(WPE,
   extrapolate_faces<N>(sQh, sFh, s, qf + cell * 6 * V * B2, ff + cell * 6 * V * B2);
   if (s == 0) {
     if (iters) iters[cell] = it;
-    if (sweep_count) atomicAdd(sweep_count, (unsigned long long)it);
+    count_sweeps(sweep_count, cell, it);
   }
 }
 
@@ -1321,7 +1321,7 @@ __global__ __launch_bounds__(Ord<N>::NT) void k_predictor_staged(
     extrapolate_faces<N>(sQh, sFh, s, qf + cell * 6 * V * B2, ff + cell * 6 * V * B2);
     if (s == 0) {
       if (iters) iters[cell] = it;
-      if (sweep_count) atomicAdd(sweep_count, (unsigned long long)it);
+      count_sweeps(sweep_count, cell, it);
     }
   }
 }

@@ -256,7 +256,7 @@ __global__ __launch_bounds__(Ord<N>::NT) void k_predictor_pde(
   extrapolate_faces<N>(sQh, sFh, s, qf + cell * 6 * V * B2, ff + cell * 6 * V * B2);
   if (s == 0) {
     if (iters) iters[cell] = it;
-    if (sweep_count) atomicAdd(sweep_count, (unsigned long long)it);
+    count_sweeps(sweep_count, cell, it);
   }
 }
 

@@ -770,8 +770,9 @@ extern "C" int exa_amr_grid_create(exa_solver* s, const exa_amr_config* cfg, exa
   EXA_CHECK(hipMemset(g->qf.p, 0, facev));
   EXA_CHECK(hipMemset(g->ff.p, 0, facev));
   EXA_TRY(g->iters.ensure(sizeof(int) * nc));
-  EXA_TRY(g->iter_sum.ensure(sizeof(unsigned long long)));
-  EXA_CHECK(hipMemset(g->iter_sum.p, 0, sizeof(unsigned long long)));
+  EXA_TRY(g->iter_sum.ensure(EXA_SWEEP_BYTES));
+  EXA_CHECK(hipMemset(g->iter_sum.p, 0, EXA_SWEEP_BYTES));
+  EXA_CHECK(hipStreamSynchronize(nullptr));  // the grid's stream does not wait for the null stream
   EXA_TRY(up(g->face_kind, face_kind.data(), sizeof(int) * nc * 6));
   EXA_TRY(up(g->face_ref, face_ref.data(), sizeof(int) * nc * 6));
   EXA_TRY(up(g->anc_kids, anc_kids.data(), sizeof(int) * anc_kids.size()));
@@ -1028,9 +1029,5 @@ extern "C" int exa_amr_grid_phase_times(exa_amr_grid* g, double ms[6], long long
 extern "C" int exa_amr_grid_total_picard_iterations(exa_amr_grid* g, long long* total) {
   EXA_ARG(g && total, "null pointer");
   EXA_CHECK(hipSetDevice(g->device));
-  EXA_CHECK(hipStreamSynchronize(g->stream));
-  unsigned long long t = 0;
-  EXA_CHECK(hipMemcpy(&t, g->iter_sum.p, sizeof(t), hipMemcpyDeviceToHost));
-  *total = (long long)t;
-  return EXA_OK;
+  return exa_read_sweeps(g->iter_sum.as<unsigned long long>(), false, g->stream, total);
 }

@@ -1121,7 +1121,8 @@ struct exa_grid {
   double* dt_cur() const { return state.as<double>(); }
   unsigned long long* dt_next() const { return reinterpret_cast<unsigned long long*>(state.as<double>() + 1); }
   double* time() const { return state.as<double>() + 2; }
-  unsigned long long* iter_sum() const { return reinterpret_cast<unsigned long long*>(state.as<double>() + 3); }
+  DevBuf sweeps;  // sweep counter
+  unsigned long long* iter_sum() const { return sweeps.as<unsigned long long>(); }
   double* dt_pred() const { return state.as<double>() + 4; }  // fused stepping: the optimistic dt
   unsigned long long* reruns() const { return reinterpret_cast<unsigned long long*>(state.as<double>() + 5); }
 };
@@ -1187,7 +1188,7 @@ extern "C" int exa_grid_create(exa_solver* s, int nx, int ny, int nz, const doub
       (r = g->qf.ensure(sizeof(double) * g->nc * 6 * V * B2)) != EXA_OK ||
       (r = g->ff.ensure(sizeof(double) * g->nc * 6 * V * B2)) != EXA_OK ||
       (r = g->iters.ensure(sizeof(int) * g->nc)) != EXA_OK || (r = g->nbr.ensure(sizeof(int) * 6 * g->nc)) != EXA_OK ||
-      (r = g->state.ensure(sizeof(double) * 8)) != EXA_OK) {
+      (r = g->state.ensure(sizeof(double) * 8)) != EXA_OK || (r = g->sweeps.ensure(EXA_SWEEP_BYTES)) != EXA_OK) {
     delete g;
     return r;
   }
@@ -1205,6 +1206,8 @@ extern "C" int exa_grid_create(exa_solver* s, int nx, int ny, int nz, const doub
   std::memcpy(&st[1], &big, sizeof(big));
   if (e == hipSuccess) e = hipMemcpy(g->state.p, st, sizeof(st), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemset(g->iters.p, 0, sizeof(int) * g->nc);
+  if (e == hipSuccess) e = hipMemset(g->sweeps.p, 0, EXA_SWEEP_BYTES);
+  if (e == hipSuccess) e = hipStreamSynchronize(nullptr);  // the grid's stream does not wait for the null stream
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking);
   if (e != hipSuccess) {
     exa_set_error("grid setup: %s", hipGetErrorString(e));
@@ -1692,12 +1695,7 @@ extern "C" int exa_grid_picard_iterations(exa_grid* g, int* iters) {
 extern "C" int exa_grid_total_picard_iterations(exa_grid* g, long long* total) {
   EXA_ARG(g && total, "null pointer");
   EXA_CHECK(hipSetDevice(g->s->device));
-  unsigned long long h = 0, zero = 0;
-  EXA_CHECK(hipMemcpyAsync(&h, g->iter_sum(), sizeof(h), hipMemcpyDeviceToHost, g->stream));
-  EXA_CHECK(hipMemcpyAsync(g->iter_sum(), &zero, sizeof(zero), hipMemcpyHostToDevice, g->stream));
-  EXA_CHECK(hipStreamSynchronize(g->stream));
-  *total = (long long)h;
-  return EXA_OK;
+  return exa_read_sweeps(g->iter_sum(), true, g->stream, total);
 }
 
 extern "C" int exa_grid_kernel_times(exa_grid* g, double times[3], long long counts[3]) {
@@ -1854,7 +1852,7 @@ extern "C" int exa_ensemble_create(const exa_ensemble_member* m, int n, const ex
         (r = gr->cell_inst.ensure(sizeof(int) * gr->nc)) != EXA_OK ||
         (r = gr->params.ensure(sizeof(exa::InstParams) * mem.size())) != EXA_OK ||
         (r = gr->ics.ensure(sizeof(exa_ic) * mem.size())) != EXA_OK ||
-        (r = gr->iter_sum.ensure(sizeof(unsigned long long))) != EXA_OK) {
+        (r = gr->iter_sum.ensure(EXA_SWEEP_BYTES)) != EXA_OK) {
       exa_ensemble_destroy(e);
       return r;
     }
@@ -1879,7 +1877,8 @@ extern "C" int exa_ensemble_create(const exa_ensemble_member* m, int n, const ex
     if (he == hipSuccess)
       he = hipMemcpy(gr->params.p, gr->hp.data(), sizeof(exa::InstParams) * gr->hp.size(), hipMemcpyHostToDevice);
     if (he == hipSuccess) he = hipMemset(gr->iters.p, 0, sizeof(int) * gr->nc);
-    if (he == hipSuccess) he = hipMemset(gr->iter_sum.p, 0, sizeof(unsigned long long));
+    if (he == hipSuccess) he = hipMemset(gr->iter_sum.p, 0, EXA_SWEEP_BYTES);
+    if (he == hipSuccess) he = hipStreamSynchronize(nullptr);  // as for a grid
     if (he != hipSuccess) {
       exa_set_error("ensemble setup: %s", hipGetErrorString(he));
       exa_ensemble_destroy(e);
@@ -2040,10 +2039,9 @@ extern "C" int exa_ensemble_total_picard_iterations(exa_ensemble* e, long long* 
   EXA_CHECK(hipStreamSynchronize(e->stream));
   long long t = 0;
   for (EnsGroup* gr : e->groups) {
-    unsigned long long h = 0, zero = 0;
-    EXA_CHECK(hipMemcpy(&h, gr->iter_sum.p, sizeof(h), hipMemcpyDeviceToHost));
-    EXA_CHECK(hipMemcpy(gr->iter_sum.p, &zero, sizeof(zero), hipMemcpyHostToDevice));
-    t += (long long)h;
+    long long h = 0;
+    EXA_TRY(exa_read_sweeps(gr->iter_sum.as<unsigned long long>(), true, e->stream, &h));
+    t += h;
   }
   *total = t;
   return EXA_OK;

@@ -64,6 +64,20 @@ struct DevBuf {
   }
 };
 
+// Sum of a sweep counter (EXA_SWEEP_SLOTS words), cleared if asked for; waits
+// for the stream.
+static inline int exa_read_sweeps(unsigned long long* count, bool clear, hipStream_t stream, long long* total) {
+  unsigned long long h[EXA_SWEEP_SLOTS * EXA_SWEEP_STRIDE];
+  EXA_CHECK(hipMemcpyAsync(h, count, sizeof(h), hipMemcpyDeviceToHost, stream));
+  EXA_CHECK(hipStreamSynchronize(stream));
+  *total = 0;
+  for (int i = 0; i < EXA_SWEEP_SLOTS; ++i) *total += (long long)h[i * EXA_SWEEP_STRIDE];
+  if (!clear) return EXA_OK;
+  EXA_CHECK(hipMemsetAsync(count, 0, sizeof(h), stream));
+  EXA_CHECK(hipStreamSynchronize(stream));
+  return EXA_OK;
+}
+
 static inline unsigned long long exa_big_bits() {
   const double big = 1.0e300;
   unsigned long long b;
