@@ -1,4 +1,4 @@
-// Space-time predictor of the Euler equations at orders 4..8, FP64 and mixed
+// Space-time predictor of the Euler equations at orders 1..8, FP64 and mixed
 // precision (the default form): Picard iteration, time averages, volume
 // integral and face extrapolation of one cell per workgroup.  Same scheme as
 // k_predictor (spaceTimePredictorNonlinear.cpph:43-577,
@@ -12,6 +12,9 @@
 // constants (the scale is applied once per node), and 180 instead of 254
 // registers at N = 5 (pin, park).  ms per launch (FP64 / FP32 sweeps, vortex
 // grid; before: the fastest of the other forms):
+//   N = 1  45^3   0.42 -> 0.23     0.45 -> 0.23
+//   N = 2  45^3   0.72 -> 0.48     0.68 -> 0.40
+//   N = 3  45^3   1.23 -> 0.81     1.07 -> 0.66
 //   N = 4  45^3   2.84 -> 1.78     2.50 -> 1.51
 //   N = 5  45^3   6.05 -> 4.07     5.69 -> 3.50
 //   N = 6  27^3   3.86 -> 2.26     3.48 -> 1.94
@@ -85,8 +88,9 @@ struct HistOrd {
   // (spills), mixed 4.5 / 3.65 / 3.8.  N = 6 is six waves per workgroup, of
   // which two fit only at 4 per SIMD: FP64 spills there (2.3 / - / 3.9 at
   // 27^3), mixed does not (2.1 / 2.1 / 1.9).  N = 7: 3.4 / 4.7 and 2.9 / 3.5.
-  static constexpr int WPE64 = N == 6 || N == 7 ? 2 : 3;
-  static constexpr int WPEMX = N == 7 ? 2 : N == 6 ? 4 : 3;
+  // N = 3 (one wave per cell): 0.88 / 0.81 / 0.81 and 0.78 / 0.68 / 0.66.
+  static constexpr int WPE64 = N <= 3 ? 4 : N == 6 || N == 7 ? 2 : 3;
+  static constexpr int WPEMX = N == 7 ? 2 : N <= 3 || N == 6 ? 4 : 3;
   static constexpr int lds_doubles(bool fp64_sweeps, bool one_sweep) {
     const int p = fp64_sweeps ? PARK64 * V * Ord<N>::B3 : 0;
     const int q = one_sweep ? (PARKMX * V * Ord<N>::B3 + 1) / 2 : 0;

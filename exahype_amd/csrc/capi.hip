@@ -277,10 +277,9 @@ static bool predictor_staged(const exa_aderdg_config& c, int dev) {
 }
 
 // The default predictor of the Euler equations in FP64 or with FP32 sweeps
-// (pred_history.hip; faster than every other form at orders 4..8, see
+// (pred_history.hip; faster than every other form at orders 1..8, see
 // aderdg_history.h), unless the configuration or exa_autotune asks for another
-// form.  Below, cells are too small for it to matter (N = 3, 45^3 cells: 1.16
-// against 1.25 ms FP64, 1.37 against 1.14 mixed); at order 9 its registers do not hold
+// form.  At order 9 its registers do not hold
 // the state (7.8 ms against the staged form's 6.8 at 18^3 cells, FP64).
 static bool predictor_history(const exa_aderdg_config& c, int dev) {
   return c.pde == EXA_PDE_EULER && !c.linear && c.order >= EXA_HISTORY_MIN_ORDER &&

@@ -1,4 +1,4 @@
-// The default Euler predictors (aderdg_history.h), orders 4..8: FP64, FP32
+// The default Euler predictors (aderdg_history.h), orders 1..8: FP64, FP32
 // sweeps before the FP64 correction sweeps, and the latter's variant for
 // meshes with many uniform cells (orders up to 7, the adaptive mesh's range).
 #include "aderdg_history.h"
@@ -20,6 +20,9 @@ PredFn pick(bool mixed, int fp64_sweeps, bool uskip) {
 
 PredFn exa_pred_history_kernel(int order, bool mixed, int fp64_sweeps, bool uskip) {
   switch (order) {
+    case 1: return pick<1>(mixed, fp64_sweeps, uskip);
+    case 2: return pick<2>(mixed, fp64_sweeps, uskip);
+    case 3: return pick<3>(mixed, fp64_sweeps, uskip);
     case 4: return pick<4>(mixed, fp64_sweeps, uskip);
     case 5: return pick<5>(mixed, fp64_sweeps, uskip);
     case 6: return pick<6>(mixed, fp64_sweeps, uskip);
@@ -39,6 +42,9 @@ int lds_bytes(bool fp64_sweeps, bool one_sweep) {
 int exa_pred_history_lds_bytes(int order, bool mixed, int fp64_sweeps, bool uskip) {
   const bool one = mixed && fp64_sweeps == 1, f64 = !one || uskip;  // the sweeps that the kernel holds
   switch (order) {
+    case 1: return lds_bytes<1>(f64, one);
+    case 2: return lds_bytes<2>(f64, one);
+    case 3: return lds_bytes<3>(f64, one);
     case 4: return lds_bytes<4>(f64, one);
     case 5: return lds_bytes<5>(f64, one);
     case 6: return lds_bytes<6>(f64, one);

@@ -33,10 +33,10 @@ EXA_PRED_TU_DECL(6)
 EXA_PRED_TU_DECL(7)
 #undef EXA_PRED_TU_DECL
 
-// The default of the Euler equations at orders 4..8 (pred_history.hip):
+// The default of the Euler equations at orders 1..8 (pred_history.hip):
 // FP64, or FP32 sweeps before the FP64 correction sweeps (mixed); uskip as
 // above (mixed, orders up to 7; ignored otherwise).
-#define EXA_HISTORY_MIN_ORDER 4
+#define EXA_HISTORY_MIN_ORDER 1
 #define EXA_HISTORY_MAX_ORDER 8
 PredFn exa_pred_history_kernel(int order, bool mixed, int fp64_sweeps, bool uskip = false);
 int exa_pred_history_lds_bytes(int order, bool mixed, int fp64_sweeps, bool uskip = false);
