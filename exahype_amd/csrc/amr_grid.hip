@@ -188,6 +188,7 @@ struct exa_amr_grid {
   exa_solver* s = nullptr;
   exa_amr_config cfg{};
   int device = 0, N = 0, B = 0, P = 0, S = 0, levels = 1, finest = 0;
+  HostStage hstage;
   hipStream_t stream = nullptr;
   std::vector<Leaf> leaves;
   long long nc = 0, first_fine = 0, nslots = 0, nfaces = 0, cap = 0;
@@ -852,13 +853,8 @@ extern "C" int exa_amr_grid_cells(const exa_amr_grid* g, int* cells) {
 extern "C" int exa_amr_grid_upload(exa_amr_grid* g, const double* luh) {
   EXA_ARG(g && luh, "null pointer");
   EXA_CHECK(hipSetDevice(g->device));
-  const int B3 = g->B * g->B * g->B;
-  std::vector<double> h((size_t)g->nc * V * B3);
-  for (long long q = 0; q < g->nc; ++q)
-    for (int n = 0; n < B3; ++n)
-      for (int v = 0; v < V; ++v) h[(size_t)q * V * B3 + v * B3 + n] = luh[((size_t)q * B3 + n) * V + v];
-  EXA_CHECK(hipStreamSynchronize(g->stream));
-  EXA_CHECK(hipMemcpy(g->luh.p, h.data(), sizeof(double) * h.size(), hipMemcpyHostToDevice));
+  EXA_TRY(exa_transfer_nodes(g->hstage, g->stream, g->luh.as<double>(), const_cast<double*>(luh), g->nc,
+                             g->B * g->B * g->B, true));
   g->dt_valid = false;
   return limiter_start(g, nullptr);
 }
@@ -866,14 +862,7 @@ extern "C" int exa_amr_grid_upload(exa_amr_grid* g, const double* luh) {
 extern "C" int exa_amr_grid_download(exa_amr_grid* g, double* luh) {
   EXA_ARG(g && luh, "null pointer");
   EXA_CHECK(hipSetDevice(g->device));
-  EXA_CHECK(hipStreamSynchronize(g->stream));
-  const int B3 = g->B * g->B * g->B;
-  std::vector<double> h((size_t)g->nc * V * B3);
-  EXA_CHECK(hipMemcpy(h.data(), g->luh.p, sizeof(double) * h.size(), hipMemcpyDeviceToHost));
-  for (long long q = 0; q < g->nc; ++q)
-    for (int n = 0; n < B3; ++n)
-      for (int v = 0; v < V; ++v) luh[((size_t)q * B3 + n) * V + v] = h[(size_t)q * V * B3 + v * B3 + n];
-  return EXA_OK;
+  return exa_transfer_nodes(g->hstage, g->stream, g->luh.as<double>(), luh, g->nc, g->B * g->B * g->B, false);
 }
 
 extern "C" int exa_amr_grid_set_initial_conditions(exa_amr_grid* g, const exa_ic* ic) {

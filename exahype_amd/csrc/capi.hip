@@ -1103,6 +1103,7 @@ struct exa_grid {
   int nb = 0;
   DevBuf bfaces, bq, bf;
   DevBuf sample;   // Cartesian-vertex samples (output)
+  HostStage hstage;
   int nslots = 0;
   bool staged = false;  // decided at creation (the slots are allocated then)
   hipStream_t stream = nullptr;
@@ -1260,39 +1261,19 @@ extern "C" int exa_grid_num_cells(const exa_grid* g, long long* n) {
   return EXA_OK;
 }
 
-static int grid_transfer(exa_grid* g, double* host, bool upload) {
-  const int B = g->s->cfg.order + 1, B3 = B * B * B, V = exa::V;
-  const size_t per = (size_t)V * B3;
-  const long long chunk = 4096;
-  std::vector<double> buf(per * chunk);
-  for (long long c0 = 0; c0 < g->nc; c0 += chunk) {
-    const long long n = std::min(chunk, g->nc - c0);
-    double* dev = g->luh.as<double>() + c0 * per;
-    if (upload) {
-      for (long long c = 0; c < n; ++c) ref_to_soa_cell(host + (c0 + c) * per, buf.data() + c * per, B3, V);
-      EXA_CHECK(hipMemcpyAsync(dev, buf.data(), sizeof(double) * per * n, hipMemcpyHostToDevice, g->stream));
-      EXA_CHECK(hipStreamSynchronize(g->stream));
-    } else {
-      EXA_CHECK(hipMemcpyAsync(buf.data(), dev, sizeof(double) * per * n, hipMemcpyDeviceToHost, g->stream));
-      EXA_CHECK(hipStreamSynchronize(g->stream));
-      for (long long c = 0; c < n; ++c) soa_to_ref_cell(buf.data() + c * per, host + (c0 + c) * per, B3, V);
-    }
-  }
-  return EXA_OK;
-}
-
 extern "C" int exa_grid_upload(exa_grid* g, const double* luh) {
   EXA_ARG(g && luh, "null pointer");
   EXA_CHECK(hipSetDevice(g->s->device));
   ++g->version;
-  return grid_transfer(g, const_cast<double*>(luh), true);
+  const int B = g->s->cfg.order + 1;
+  return exa_transfer_nodes(g->hstage, g->stream, g->luh.as<double>(), const_cast<double*>(luh), g->nc, B * B * B, true);
 }
 
 extern "C" int exa_grid_download(exa_grid* g, double* luh) {
   EXA_ARG(g && luh, "null pointer");
   EXA_CHECK(hipSetDevice(g->s->device));
-  EXA_CHECK(hipStreamSynchronize(g->stream));
-  return grid_transfer(g, luh, false);
+  const int B = g->s->cfg.order + 1;
+  return exa_transfer_nodes(g->hstage, g->stream, g->luh.as<double>(), luh, g->nc, B * B * B, false);
 }
 
 extern "C" int exa_grid_sample_cartesian(exa_grid* g, double* out) {
@@ -1743,6 +1724,7 @@ struct exa_ensemble {
   bool dt_valid = false;  // exa_ensemble_compute_dt has run (sync checks the dts from then on)
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
+  HostStage hstage;
 };
 
 static exa::Ens ens_of(EnsGroup* gr) {
@@ -2020,16 +2002,11 @@ extern "C" int exa_ensemble_sync(exa_ensemble* e, double* times, double* dts) {
 extern "C" int exa_ensemble_download(exa_ensemble* e, int instance, double* luh) {
   EXA_ARG(e && luh && instance >= 0 && instance < (int)e->where.size(), "instance");
   EXA_CHECK(hipSetDevice(e->device));
-  EXA_CHECK(hipStreamSynchronize(e->stream));
   EnsGroup* gr = e->groups[e->where[instance].first];
   const exa::InstParams& p = gr->hp[e->where[instance].second];
-  const int B = gr->order + 1, B3 = B * B * B, V = exa::V;
-  const size_t per = (size_t)V * B3, nci = (size_t)p.nx * p.ny * p.nz;
-  std::vector<double> buf(per * nci);
-  EXA_CHECK(hipMemcpy(buf.data(), gr->luh.as<double>() + p.base * per, sizeof(double) * buf.size(),
-                      hipMemcpyDeviceToHost));
-  for (size_t c = 0; c < nci; ++c) soa_to_ref_cell(buf.data() + c * per, luh + c * per, B3, V);
-  return EXA_OK;
+  const int B = gr->order + 1, B3 = B * B * B;
+  return exa_transfer_nodes(e->hstage, e->stream, gr->luh.as<double>() + (size_t)p.base * exa::V * B3, luh,
+                            (long long)p.nx * p.ny * p.nz, B3, false);
 }
 
 extern "C" int exa_ensemble_total_picard_iterations(exa_ensemble* e, long long* total) {

@@ -215,6 +215,7 @@ struct exa_fv_grid {
   int nx = 1, ny = 1, nz = 1, np = 0;
   double off[3] = {0, 0, 0}, width[3] = {1, 1, 1}, dx[3] = {1, 1, 1};
   DevBuf cur, nxt, nbr, state;
+  HostStage hstage;
   int periodic[3] = {1, 1, 1};  // closed axes take the boundary values bc
   exa_bc bc{};
   hipStream_t stream = nullptr;
@@ -465,18 +466,7 @@ extern "C" int exa_fv_grid_kernel_times(exa_fv_grid* g, double times[4], long lo
 }
 
 static int fv_grid_transfer(exa_fv_grid* g, double* host, bool upload) {
-  const int nbox = g->s->geom().ncells_box();
-  const size_t psz = (size_t)nbox * FV_V;
-  std::vector<double> buf(psz * g->np);
-  if (upload) {
-    for (int p = 0; p < g->np; ++p) patch_ref_to_soa(host + p * psz, buf.data() + p * psz, nbox);
-    EXA_CHECK(hipMemcpy(g->cur.p, buf.data(), sizeof(double) * buf.size(), hipMemcpyHostToDevice));
-  } else {
-    EXA_CHECK(hipStreamSynchronize(g->stream));
-    EXA_CHECK(hipMemcpy(buf.data(), g->cur.p, sizeof(double) * buf.size(), hipMemcpyDeviceToHost));
-    for (int p = 0; p < g->np; ++p) patch_soa_to_ref(buf.data() + p * psz, host + p * psz, nbox);
-  }
-  return EXA_OK;
+  return exa_transfer_nodes(g->hstage, g->stream, g->cur.as<double>(), host, g->np, g->s->geom().ncells_box(), upload);
 }
 
 extern "C" int exa_fv_grid_upload(exa_fv_grid* g, const double* luh) {

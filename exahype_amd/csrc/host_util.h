@@ -64,6 +64,23 @@ struct DevBuf {
   }
 };
 
+// Two pinned buffers and their events, kept by the object whose solution they
+// move (at most 8 MB each, or one cell block), allocated by its first transfer.
+struct HostStage {
+  double* buf[2] = {nullptr, nullptr};
+  hipEvent_t ev[2] = {nullptr, nullptr};
+  size_t words = 0;  // of each buffer
+  HostStage() = default;
+  HostStage(const HostStage&) = delete;
+  HostStage& operator=(const HostStage&) = delete;
+  ~HostStage();
+  bool ensure(size_t n);  // false: no memory
+};
+// units blocks [v][node] on the device from (up) or to user's [node][v] in
+// host memory, behind the work queued on the stream; complete on return.
+int exa_transfer_nodes(HostStage& st, hipStream_t stream, double* blocks, double* user, long long units, int nodes,
+                       bool up);
+
 // Sum of a sweep counter (EXA_SWEEP_SLOTS words), cleared if asked for; waits
 // for the stream.
 static inline int exa_read_sweeps(unsigned long long* count, bool clear, hipStream_t stream, long long* total) {

@@ -1,0 +1,66 @@
+"""Uploads and downloads through the pinned buffers: every value at its place,
+bit for bit, for one short chunk, many chunks with a short last one, single
+cells larger than usual, special values, and a transfer behind queued steps."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("N,n", [(1, (1, 1, 1)), (3, (2, 3, 5)), (2, (31, 30, 29)), (5, (11, 10, 9)), (9, (9, 8, 7))])
+def test_grid_roundtrip(N, n):
+    import exahype_amd as E
+    g = E.Grid(E.ADERDGSolver(N), *n)
+    a = np.random.default_rng(N).standard_normal(g.ncells * g.cell_size)
+    a[:6] = (np.nan, np.inf, -np.inf, -0.0, 5e-324, 1e308)[:6]
+    for k in range(2):  # the second transfer finds the buffers of the first
+        g.upload(a + k)
+        assert np.array_equal(g.download().view(np.int64), (a + k).view(np.int64))
+
+
+@pytest.mark.parametrize("dim,P,n", [(2, 10, (7, 5, 1)), (3, 3, (4, 3, 2)), (3, 11, (5, 4, 4))])
+def test_fv_roundtrip(dim, P, n):
+    import exahype_amd as E
+    s = E.FiniteVolumesSolver(dim, P, scheme=E.FV_GODUNOV if dim == 2 else E.FV_MUSCLHANCOCK)
+    g = E.FVGrid(s, *n)
+    a = np.random.default_rng(P).standard_normal(g.npatch * s.patch_size)
+    g.upload(a)
+    assert np.array_equal(g.download(), a)
+
+
+def test_layout_and_order_behind_steps():
+    """Device blocks are [v][node]: the initial conditions read back are the
+    per-cell entry point's; a download waits for the steps before it."""
+    import exahype_amd as E
+    s = E.ADERDGSolver(4)
+    ic = E.make_ic(5, xc=(0.4, 0.5, 0.6), L=0.05, amp=0.3, rho_inf=1.0, p_inf=1.0, uinf=(0.4, -0.3, 0.2))
+    g = E.Grid(s, 12, 11, 10)
+    g.set_initial_conditions(ic)
+    cells = g.download().reshape(g.ncells, -1)
+    dx = np.array([1 / 12, 1 / 11, 1 / 10])
+    for c in (0, 13, g.ncells - 1):
+        i = np.array([c % 12, c // 12 % 11, c // 132])
+        assert np.array_equal(cells[c], s.adjustSolution((i + 0.5) * dx, dx, 0.0, ic))
+    g.compute_dt()
+    g.use_graph(True)
+    g.step(20)
+    a = g.download()
+    g.sync()
+    assert np.array_equal(a, g.download()) and not np.array_equal(a, cells.ravel())
+
+
+def test_adaptive_grid_and_ensemble():
+    import exahype_amd as E
+    s = E.ADERDGSolver(3)
+    g = E.AMRGrid(s, E.amr_config(3, 2, (0.5, 0.5, 0.5), 0.25, (0.1,)))
+    a = np.tile(np.array((1.0, 0.1, -0.2, 0.3, 2.5)), g.ncells * 64)
+    a *= 1 + 0.01 * np.random.default_rng(0).random(a.size)
+    g.upload(a)
+    assert np.array_equal(g.download(), a)
+    ic = E.make_ic(5, xc=(0.4, 0.5, 0.6), L=0.05, amp=0.3, rho_inf=1.0, p_inf=1.0, uinf=(0.4, -0.3, 0.2))
+    e = E.Ensemble([dict(order=n, cells=(4, 5, 3)) for n in (2, 4, 4)])
+    e.set_initial_conditions([ic] * 3)
+    for i, n in enumerate((2, 4, 4)):
+        o = E.Grid(E.ADERDGSolver(n), 4, 5, 3)
+        o.set_initial_conditions(ic)
+        assert np.array_equal(e.download(i), o.download())
