@@ -282,7 +282,6 @@ size_t proj_lds(int B) {
   const int L = 2 * B - 1;
   return sizeof(double) * (size_t)V * (B * B * L + B * L * L);  // lim::proj_t_lds_doubles<B>
 }
-size_t muscl_lds(int P) { return sizeof(double) * V * (size_t)P * P * P; }
 
 // ---- the limiter's starting state (setInitialConditions, then the status
 // after them: admissibility only, LimitingADERDGSolver.cpp:906-930)
@@ -502,8 +501,9 @@ int enqueue_step(exa_amr_grid* g, int par, bool timed) {
       constexpr int PP = decltype(p)::value;
       hipLaunchKernelGGL(k_ghost_fill<PP>, dim3(capb), dim3(256), 0, g->stream, pool_old, g->list_cells(k),
                          g->list_slots(k), g->count(k), g->slot_of.as<int>(), st, g->nbr6.as<int>(), cnt);
-      hipLaunchKernelGGL(k_muscl_list<PP>, dim3(capb), dim3(256), muscl_lds(PP), g->stream, pool_old, pool_new,
-                         g->list_slots(k), g->count(k), hf, g->ip(), g->finest, gamma);
+      hipLaunchKernelGGL(k_muscl_list<PP>, dim3(capb), dim3(exa::fv::MusclForm<PP>::NT),
+                         exa::fv::MusclForm<PP>::LDS, g->stream, pool_old, pool_new, g->list_slots(k), g->count(k), hf,
+                         g->ip(), g->finest, gamma);
     }));
     EXA_TRY(with_patch(P, [&](auto p) {
       constexpr int PP = decltype(p)::value;
@@ -814,7 +814,7 @@ extern "C" int exa_amr_grid_create(exa_solver* s, const exa_amr_config* cfg, exa
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)proj_lds(g->B));
     if (e == hipSuccess)
       e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_muscl_list<PP>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)muscl_lds(PP));
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)exa::fv::MusclForm<PP>::LDS);
   }));
   EXA_CHECK(e);
   EXA_CHECK(hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking));

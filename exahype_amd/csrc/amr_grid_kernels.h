@@ -314,16 +314,16 @@ __global__ __launch_bounds__(256) void k_ghost_fill(double* __restrict__ pool, c
 
 // MUSCL-Hancock update of the listed patches: old pool -> new pool.
 template <int P>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(fv::muscl_min_waves(P)))) void k_muscl_list(const double* __restrict__ pool_old, double* __restrict__ pool_new,
-                                                    const int* __restrict__ slots, const int* __restrict__ count,
-                                                    double dx, const InstParams* __restrict__ inst, int level,
-                                                    double gamma) {
+__global__ __launch_bounds__(fv::MusclForm<P>::NT)
+    __attribute__((amdgpu_waves_per_eu(3))) void k_muscl_list(
+        const double* __restrict__ pool_old, double* __restrict__ pool_new, const int* __restrict__ slots,
+        const int* __restrict__ count, double dx, const InstParams* __restrict__ inst, int level, double gamma) {
   if ((int)blockIdx.x >= *count) return;
-  extern __shared__ double sQt[];
+  extern __shared__ double sm[];
   constexpr int S3 = (P + 4) * (P + 4) * (P + 4);
   const size_t o = (size_t)slots[blockIdx.x] * V * S3;
   // the kernel's own CFL (kernels/finitevolumes/musclhancock/c/musclhancock.h:29)
-  fv::muscl_patch<EulerPDE, P>(pool_old + o, pool_new + o, sQt, dx, dx, dx, inst[level].dt_cur, gamma, 0.99);
+  fv::muscl_patch<EulerPDE, P>(pool_old + o, pool_new + o, sm, dx, dx, dx, inst[level].dt_cur, gamma, 0.99);
 }
 
 // DG <-> FV projections of the listed cells (Limiter.cpp:23-112).

@@ -144,149 +144,284 @@ __global__ __launch_bounds__(256) void k_godunov(const double* __restrict__ luh,
 }
 
 __device__ inline double minmod(double a, double b) {
-  if (a * b < 0.0) return 0.0;
-  return fabs(a) < fabs(b) ? a : b;
+  const double m = fabs(a) < fabs(b) ? a : b;
+  return a * b < 0.0 ? 0.0 : m;
+}
+
+// Admissible time step of faces with wave speeds s: the smallest exa_dt_sane(
+// cfl_h / s), with one division for the largest speed instead of one a face.
+struct FaceSpeeds {
+  double hi = 0.0;
+  bool bad = false;
+  // a face with wave speed s, if `face`
+  __device__ inline void add(bool face, double s, double cfl_h) {
+    hi = face && s > hi ? s : hi;
+    if (face && !(s > 1.0e-290 && s <= 1.7976931348623157e308)) bad = bad || exa_dt_sane(cfl_h / s) == 0.0;
+  }
+  __device__ inline double candidate(double cfl_h) const {
+    return bad ? 0.0 : (hi > 0.0 ? exa_dt_sane(cfl_h / hi) : 1.0e300);
+  }
+};
+
+// A value is formed here, and not at its first use.
+__device__ inline void fv_pin(double& x) { asm volatile("" : "+v"(x)); }
+
+// The same value in every lane, held in scalar registers.
+__device__ inline double wave_uniform(double x) {
+  const long long b = __double_as_longlong(x);
+  const unsigned lo = __builtin_amdgcn_readfirstlane((int)b), hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
 // MUSCL-Hancock (kernels/finitevolumes/musclhancock/c/3d/musclhancock.cpph:
-// 27-309), one workgroup per patch, one launch:
-//   phase 1  every interior subcell evaluates its half-step evolution term
-//            Qt = sum_d (F_d(w_L,d) - F_d(w_R,d)) / h_d from its minmod slopes
-//            and boundary-extrapolated states (:62-213) into LDS;
-//   phase 2  every interior subcell rebuilds the evolved states of the faces it
-//            touches -- its own and its neighbours' w = q -+ h/2 slope, plus
-//            dt/2 Qt where the owner is interior -- and applies the Rusanov
-//            fluxes on (w_R[i], w_L[i+1]) (:215-281); the first ghost layer
-//            receives the patch-boundary face updates as in the reference,
-//            from the interior subcell next to it, which has just formed
-//            that face's flux for its own update.
-// The states are recomputed from the patch values instead of being stored
-// (six state arrays per patch would be 6x the patch's HBM traffic); they are
-// the same operations on the same inputs, hence the same values.
-__device__ inline void muscl_face_state(const double* u, int nbox, const PatchGeom& g, const double* sQt, int idx,
-                                        int d, int side, double h, double dt, double* w) {
-  double q[V], qm[V], qp[V];
-  load_q(u, nbox, idx, q);
-  load_q(u, nbox, idx - g.stride(d), qm);
-  load_q(u, nbox, idx + g.stride(d), qp);
-#pragma unroll
-  for (int v = 0; v < V; ++v) {
-    const double slope = minmod(qp[v] - q[v], q[v] - qm[v]) / h;
-    w[v] = side ? q[v] + 0.5 * h * slope : q[v] - 0.5 * h * slope;
-  }
-  const int i = idx % g.S, j = (idx / g.S) % g.S, k = idx / (g.S * g.S);
-  const int b = g.G, e = g.G + g.P;
-  if (i >= b && i < e && j >= b && j < e && k >= b && k < e) {
-    const int ci = ((k - b) * g.P + (j - b)) * g.P + (i - b), ni = g.P * g.P * g.P;
-#pragma unroll
-    for (int v = 0; v < V; ++v) w[v] += 0.5 * dt * sQt[v * ni + ci];
-  }
-}
+// 27-309), one workgroup per patch, which walks along z.  A thread owns a
+// column (x, y) of the interior or of the first ghost layer beside it and per
+// plane
+//   -  forms its slopes, the half-step evolution (:62-213; ghosts keep their
+//      unevolved states) and its six face states, once;
+//   -  exchanges the lower x and y states through the LDS, forms the fluxes of
+//      its upper x and y faces, exchanges those; the z states and fluxes stay
+//      with it from plane to plane (:215-281).
+// The first ghost layer receives the patch-boundary face updates as in the
+// reference.  The planes above are loaded while a plane is worked on.
+//
+// Bound by vector FP64 and its latencies: about 1000 instructions a plane and
+// wave (15 divisions, 6 square roots), two barriers between at most five
+// waves.  36 KB of LDS at 11^3 let four workgroups share a compute unit, and
+// cover each other's waits, if 168 registers hold a thread: values that wait
+// longest stay in the LDS or are loaded again, since a spilled register's
+// reload also waits for every load in flight (24 spills: 344 us).
+// 12 x 13 x 14 patches of 11^3: 232 us.  Forming the states of each subcell
+// and face where they are used, every state four times: 527; one thread per
+// two subcells, a patch's states in the LDS at once, one workgroup per compute
+// unit: 400.
+template <int PC>
+struct MusclForm {
+  static constexpr int S = PC + 4, T = PC + 2;
+  static constexpr int NT = round_up64(T * T);
+  static constexpr size_t LDS = sizeof(double) * V * (S * S + 4 * T * T);
+};
 
-// PC: subcells per direction (compile time: the index arithmetic of the
-// recomputed face states is then constant; the launch's geometry must match).
-// One patch per workgroup: u (with its ghost layers) -> un (interior and the
-// first ghost layer's face updates); sQt: V P^3 doubles of LDS.  Returns the
-// thread's part of the admissible time step.
+// One patch: u (with its ghost layers) -> un (interior and the first ghost
+// layer's face updates); sm: MusclForm<PC>::LDS bytes.  Returns the thread's
+// part of the admissible time step.
 template <class PDE, int PC>
-__device__ inline double muscl_patch(const double* __restrict__ u, double* __restrict__ un, double* sQt,
-                                     double dx0, double dx1, double dx2, double dt, double gamma, double cfl) {
-  const PatchGeom g{PC, 2, PC + 4, 3};
-  const int nbox = g.ncells_box();
-  const double h[3] = {dx0 / g.P, dx1 / g.P, dx2 / g.P};
-  const int ninterior = g.P * g.P * g.P;
-  // phase 1: half-step evolution term of every interior subcell
-  for (int c = threadIdx.x; c < ninterior; c += blockDim.x) {
-    int i, j, k;
-    interior_coords(g, c, i, j, k);
-    const int idx = box_index(g, i, j, k);
-    double q[V];
-    load_q(u, nbox, idx, q);
-    double Qt[V], F[V];
+__device__ __forceinline__ double muscl_patch(const double* __restrict__ u, double* __restrict__ un, double* sm,
+                                              double dx0, double dx1, double dx2, double dt, double gamma,
+                                              double cfl) {
+  constexpr int S = PC + 4, T = PC + 2, PL = S * S, nbox = S * PL, TT = T * T;
+  const double h[3] = {dx0 / PC, dx1 / PC, dx2 / PC};
+  const double fac[3] = {wave_uniform(dt / h[0]), wave_uniform(dt / h[1]), wave_uniform(dt / h[2])};
+  const double cfl_h[3] = {wave_uniform(cfl / 3 * h[0]), wave_uniform(cfl / 3 * h[1]), wave_uniform(cfl / 3 * h[2])};
+  double* sP = sm;            // [v][y][x]: the plane
+  double* sS = sP + V * PL;   // [d][v][column]: lower face states
+  double* sF = sS + 2 * V * TT;  // [d][v][column]: fluxes of the upper faces
+  // threads beyond the columns repeat column 0, a corner: same values, same places
+  const unsigned t = threadIdx.x < TT ? threadIdx.x : 0;
+  const bool column = threadIdx.x < TT;
+  const unsigned x = t % T + 1, y = t / T + 1, col = y * S + x;
+  const bool ix = column && x > 1 && x < PC + 2, iy = column && y > 1 && y < PC + 2;
+  const bool inner = ix && iy, kept = ix || iy;  // not the four corners
+  const bool up0 = iy && x < PC + 2, up1 = ix && y < PC + 2;  // a face above
+  // the columns beside this one; where there is no face, any column that has
+  // none above it (its flux is zero)
+  const bool lo0 = iy && x > 1, lo1 = ix && y > 1;
+  auto above = [&](unsigned t, int d) { return d == 0 ? (up0 ? t + 1 : t) : (up1 ? t + T : t); };
+  auto below = [&](unsigned t, int d) { return d == 0 ? (lo0 ? t - 1 : 0) : (lo1 ? t - T : 0); };
+  // the column again, so that the places derived from it are formed where they
+  // are used: a spilled one's reload waits for every load in flight
+  auto here = [&] {
+    unsigned c = t;
+    asm volatile("" : "+v"(c));
+    return c;
+  };
+  // the second ghost layer beside the faces: one node of the plane a thread
+  const bool rim = threadIdx.x < 4 * PC;
+  const unsigned side = threadIdx.x / PC, k = threadIdx.x % PC + 2;
+  const unsigned rc = !rim ? 0 : (side < 2 ? k * S + (side ? S - 1 : 0) : (side == 3 ? S - 1 : 0) * S + k);
+
+  double qm[V], q[V], qp[V], wz[V], acc[V], r[V];
+  // node c of plane z: uniform bases and one 32-bit lane offset, formed in place
+  // (left alone, the loop keeps a pointer per array and variable in registers)
+  auto offset = [](unsigned z, unsigned c) {
+    unsigned o = 8 * (z * PL + c);
+    asm volatile("" : "+v"(o));
+    return o;
+  };
+  auto load_node = [&](const double* a, unsigned z, unsigned c, double* w) {
+    const unsigned o = offset(z, c);
 #pragma unroll
-    for (int v = 0; v < V; ++v) Qt[v] = 0.0;
+    for (int v = 0; v < V; ++v)
+      w[v] = *reinterpret_cast<const double*>(reinterpret_cast<const char*>(a + v * nbox) + o);
+  };
+  auto store_node = [&](unsigned z, const double* w) {
+    const unsigned o = offset(z, col);
 #pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      double qm[V], qp[V], wL[V], wR[V];
-      load_q(u, nbox, idx - g.stride(d), qm);
-      load_q(u, nbox, idx + g.stride(d), qp);
+    for (int v = 0; v < V; ++v) *reinterpret_cast<double*>(reinterpret_cast<char*>(un + v * nbox) + o) = w[v];
+  };
+  auto put_plane = [&](const double* own) {
+#pragma unroll
+    for (int v = 0; v < V; ++v) sP[v * PL + col] = own[v];
+#pragma unroll
+    for (int v = 0; v < V; ++v) sP[v * PL + rc] = r[v];
+  };
+  FaceSpeeds speeds[3];
+  // the upper face of the plane below, whose update it completes
+  auto z_face = [&](const double* w, double* f) {
+    speeds[2].add(inner, rusanov<PDE>(wz, w, 2, gamma, f), cfl_h[2]);
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+      f[v] = inner ? fac[2] * f[v] : 0.0;
+      acc[v] -= f[v];
+    }
+  };
+  load_node(u, 0, col, r);
+  load_node(u, 1, col, qm);
+  load_node(u, 2, col, q);
+  load_node(u, 3, col, qp);
+  load_node(un, 1, col, acc);
+#pragma unroll
+  for (int v = 0; v < V; ++v) wz[v] = qm[v] + 0.5 * minmod(q[v] - qm[v], qm[v] - r[v]);
+  // between the planes the sum and the upper z state wait in this thread's own
+  // places of sS, free until the lower states are written there: 20 registers
+  // less where most are in use, which is what lets three waves a SIMD run
+  auto park = [&] {
+    const unsigned t = here();
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+      sS[v * TT + t] = acc[v];
+      sS[(V + v) * TT + t] = wz[v];
+    }
+    asm volatile("" ::: "memory");  // not kept in registers all the same
+  };
+  auto unpark = [&] {
+    const unsigned t = here();
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+      acc[v] = sS[v * TT + t];
+      wz[v] = sS[(V + v) * TT + t];
+    }
+  };
+  load_node(u, 2, rc, r);
+  put_plane(q);
+  park();
+  __syncthreads();
+#pragma unroll 1
+  for (int z = 2; z < PC + 2; ++z) {
+    double e[V], hs[3][V], f[V], w[V];
+#pragma unroll
+    for (int v = 0; v < V; ++v) e[v] = 0.0;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const int d = (i + 2) % 3, o = d == 0 ? 1 : S;
 #pragma unroll
       for (int v = 0; v < V; ++v) {
-        const double slope = minmod(qp[v] - q[v], q[v] - qm[v]) / h[d];
-        wL[v] = q[v] - 0.5 * h[d] * slope;
-        wR[v] = q[v] + 0.5 * h[d] * slope;
+        const double a = d == 2 ? qm[v] : sP[v * PL + col - o], b = d == 2 ? qp[v] : sP[v * PL + col + o];
+        hs[d][v] = 0.5 * minmod(b - q[v], q[v] - a);
+        w[v] = q[v] - hs[d][v];
       }
-      PDE::flux_dir(wL, d, F, gamma);
+      PDE::flux_dir(w, d, f, gamma);
 #pragma unroll
-      for (int v = 0; v < V; ++v) Qt[v] += F[v] / h[d];
-      PDE::flux_dir(wR, d, F, gamma);
+      for (int v = 0; v < V; ++v) {
+        e[v] += 0.5 * fac[d] * f[v];
+        w[v] = q[v] + hs[d][v];
+        fv_pin(e[v]);
+      }
+      PDE::flux_dir(w, d, f, gamma);
 #pragma unroll
-      for (int v = 0; v < V; ++v) Qt[v] -= F[v] / h[d];
+      for (int v = 0; v < V; ++v) {
+        e[v] -= 0.5 * fac[d] * f[v];
+        fv_pin(e[v]);
+      }
     }
+    unpark();
+    const unsigned c = here();
 #pragma unroll
-    for (int v = 0; v < V; ++v) sQt[v * ninterior + c] = Qt[v];
+    for (int v = 0; v < V; ++v) {
+      e[v] = inner ? q[v] + e[v] : q[v];  // evolved centre
+      sS[v * TT + c] = e[v] - hs[0][v];
+      sS[(V + v) * TT + c] = e[v] - hs[1][v];
+      w[v] = e[v] - hs[2][v];
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        hs[d][v] = e[v] + hs[d][v];  // upper face states
+        fv_pin(hs[d][v]);
+      }
+    }
+    z_face(w, f);
+    if (z > 2 ? kept : inner) store_node(z - 1, acc);
+#pragma unroll
+    for (int v = 0; v < V; ++v) wz[v] = hs[2][v];
+    __builtin_amdgcn_sched_barrier(0);
+    // used at the end of the plane only: what a ghost's update is added to, and
+    // the planes above (the next one's values again: not kept through the slopes)
+    double old[V], qn[V];
+#pragma unroll
+    for (int v = 0; v < V; ++v) acc[v] = f[v];
+    load_node(un, z, inner ? 0 : col, old);
+    load_node(u, z + 1, rc, r);
+    load_node(u, z + 1, col, qp);
+    load_node(u, z + 2, col, qn);
+    __syncthreads();
+#pragma unroll
+    for (int d = 0; d < 2; ++d) {
+      const bool face = d == 0 ? up0 : up1;
+#pragma unroll
+      for (int v = 0; v < V; ++v) w[v] = sS[(d * V + v) * TT + above(c, d)];
+      speeds[d].add(face, rusanov<PDE>(hs[d], w, d, gamma, f), cfl_h[d]);
+#pragma unroll
+      for (int v = 0; v < V; ++v) {
+        f[v] = face ? fac[d] * f[v] : 0.0;
+        acc[v] -= f[v];
+        sF[(d * V + v) * TT + c] = f[v];
+        fv_pin(acc[v]);
+      }
+    }
+    put_plane(qp);
+    __syncthreads();
+    const unsigned b0 = below(c, 0), b1 = below(c, 1);
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+      acc[v] += sF[v * TT + b0];
+      acc[v] += sF[(V + v) * TT + b1];
+      acc[v] += inner ? q[v] : old[v];
+      qm[v] = q[v];
+      q[v] = qp[v];
+      qp[v] = qn[v];
+    }
+    park();
   }
-  __syncthreads();
-  // phase 2: Rusanov fluxes of the evolved face states
+  unpark();
+  double f[V], w[V];
+#pragma unroll
+  for (int v = 0; v < V; ++v) w[v] = q[v] - 0.5 * minmod(qp[v] - q[v], q[v] - qm[v]);
+  z_face(w, f);
+  if (kept) store_node(PC + 1, acc);
+  if (inner) {
+    load_node(un, PC + 2, col, acc);
+#pragma unroll
+    for (int v = 0; v < V; ++v) acc[v] += f[v];
+    store_node(PC + 2, acc);
+  }
   double dtm = 1.0e300;
-  for (int c = threadIdx.x; c < ninterior; c += blockDim.x) {
-    int i, j, k;
-    interior_coords(g, c, i, j, k);
-    const int idx = box_index(g, i, j, k);
-    const int ijk[3] = {i, j, k};
-    double acc[V], a[V], b[V], f[V];
-    load_q(u, nbox, idx, acc);
 #pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      const double fac = dt / h[d];
-      muscl_face_state(u, nbox, g, sQt, idx - g.stride(d), d, 1, h[d], dt, a);
-      muscl_face_state(u, nbox, g, sQt, idx, d, 0, h[d], dt, b);
-      double s = rusanov<PDE>(a, b, d, gamma, f);
-      double cand = exa_dt_sane(cfl / 3 * h[d] / s);
-      dtm = cand < dtm ? cand : dtm;
-#pragma unroll
-      for (int v = 0; v < V; ++v) acc[v] += fac * f[v];
-      if (ijk[d] == g.G) {  // the lower ghost's face with this subcell
-        const int gi = idx - g.stride(d);
-#pragma unroll
-        for (int v = 0; v < V; ++v) un[v * nbox + gi] = un[v * nbox + gi] - fac * f[v];
-      }
-      muscl_face_state(u, nbox, g, sQt, idx, d, 1, h[d], dt, a);
-      muscl_face_state(u, nbox, g, sQt, idx + g.stride(d), d, 0, h[d], dt, b);
-      s = rusanov<PDE>(a, b, d, gamma, f);
-      cand = exa_dt_sane(cfl / 3 * h[d] / s);
-      dtm = cand < dtm ? cand : dtm;
-#pragma unroll
-      for (int v = 0; v < V; ++v) acc[v] -= fac * f[v];
-      if (ijk[d] == g.G + g.P - 1) {  // the upper ghost's
-        const int gi = idx + g.stride(d);
-#pragma unroll
-        for (int v = 0; v < V; ++v) un[v * nbox + gi] = un[v * nbox + gi] + fac * f[v];
-      }
-    }
-#pragma unroll
-    for (int v = 0; v < V; ++v) un[v * nbox + idx] = acc[v];
+  for (int d = 0; d < 3; ++d) {
+    const double cand = speeds[d].candidate(cfl_h[d]);
+    dtm = cand < dtm ? cand : dtm;
   }
   return dtm;
 }
 
-// Waves per SIMD the MUSCL-Hancock kernels are compiled for: up to 11^3
-// subcells three workgroups' half-step terms fit the LDS (53 KB each at
-// P = 11), and the kernel is then held to 168 VGPRs to let them all run
-// (4.33 against 4.55 ms per launch on 27^3 patches of 11^3); larger patches
-// keep the compiler's choice.
-__host__ __device__ constexpr int muscl_min_waves(int P) { return P <= 11 ? 3 : 1; }
-
 template <class PDE, int PC>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(muscl_min_waves(PC)))) void k_muscl(const double* __restrict__ luh, double* __restrict__ luh_new,
-                                               double* __restrict__ dt_patch, unsigned long long* dt_min,
-                                               PatchGeom, double dx0, double dx1, double dx2,
-                                               const double* __restrict__ dtp, double gamma, double cfl) {
-  extern __shared__ double sQt[];  // [v][interior subcell]
-  __shared__ double red[8];
+__global__ __launch_bounds__(MusclForm<PC>::NT) __attribute__((amdgpu_waves_per_eu(3))) void k_muscl(
+    const double* __restrict__ luh, double* __restrict__ luh_new, double* __restrict__ dt_patch,
+    unsigned long long* dt_min, PatchGeom, double dx0, double dx1, double dx2, const double* __restrict__ dtp,
+    double gamma, double cfl) {
+  extern __shared__ double sm[];
+  __shared__ double red[16];
   constexpr int nbox = (PC + 4) * (PC + 4) * (PC + 4);
-  double dtm = muscl_patch<PDE, PC>(luh + (size_t)blockIdx.x * V * nbox, luh_new + (size_t)blockIdx.x * V * nbox,
-                                    sQt, dx0, dx1, dx2, *dtp, gamma, cfl);
+  double dtm = muscl_patch<PDE, PC>(luh + (size_t)blockIdx.x * V * nbox, luh_new + (size_t)blockIdx.x * V * nbox, sm,
+                                  dx0, dx1, dx2, *dtp, gamma, cfl);
   dtm = block_min(dtm, red);
   if (threadIdx.x == 0) {
     if (dt_patch) dt_patch[blockIdx.x] = dtm;

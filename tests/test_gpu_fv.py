@@ -57,6 +57,31 @@ def test_patch_update_and_dt_vs_oracle(dim, patch, scheme, opde):
     assert abs(g_dt - o_dt) <= 1e-14 * o_dt
 
 
+@pytest.mark.parametrize("patch", list(range(2, 16)))
+def test_muscl_patch_sizes_vs_oracle(patch):
+    """Every patch size: columns that fill a wave exactly (6), leave most of one
+    idle (2) or need five (15); slopes of both signs and flat ones, an output
+    whose ghost layers are not the input's, three mesh widths.  The sum of a
+    subcell is taken in another order than the oracle's: a few rounding errors
+    of values of order one, far below the bar."""
+    import exahype_amd as E
+    s = E.FiniteVolumesSolver(3, patch, 1)
+    c = O.cfg(1, pde=0)
+    rng = np.random.default_rng(100 + patch)
+    luh = euler_state(rng, s.side ** 3).reshape(s.side, s.side, s.side, 5)
+    luh[:, :2] = luh[:, 1:2]  # flat rows: zero slopes
+    before = euler_state(rng, s.side ** 3).reshape(luh.shape)
+    before[2:-2, 2:-2, 2:-2] = luh[2:-2, 2:-2, 2:-2]
+    luh, before = luh.ravel(), before.ravel()
+    dx = np.array([0.05, 0.04, 0.03])
+    g_new, g_adm = s.solutionUpdate(before, luh, dx, 2e-4)
+    o_new, o_adm = O.musclhancock_update(c, patch, before, luh, dx, 2e-4, 0.99)
+    assert rel_err(g_new, o_new) <= TOL
+    assert abs(g_adm - o_adm) <= 1e-14 * o_adm
+    luh.reshape(s.side, s.side, s.side, 5)[2, 3, 2, 0] = np.nan  # an interior subcell: no admissible time step
+    assert s.solutionUpdate(before, luh, dx, 2e-4)[1] == 0.0
+
+
 @pytest.mark.parametrize("dim,opde", [(2, 2), (3, 0)])
 def test_fv_rusanov_vs_oracle(dim, opde):
     import exahype_amd as E
