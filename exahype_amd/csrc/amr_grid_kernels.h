@@ -323,7 +323,7 @@ __global__ __launch_bounds__(fv::MusclForm<P>::NT)
   constexpr int S3 = (P + 4) * (P + 4) * (P + 4);
   const size_t o = (size_t)slots[blockIdx.x] * V * S3;
   // the kernel's own CFL (kernels/finitevolumes/musclhancock/c/musclhancock.h:29)
-  fv::muscl_patch<EulerPDE, P>(pool_old + o, pool_new + o, sm, dx, dx, dx, inst[level].dt_cur, gamma, 0.99);
+  fv::muscl_patch<EulerPDE, P, false>(pool_old + o, pool_new + o, sm, dx, dx, dx, inst[level].dt_cur, gamma, 0.99);
 }
 
 // DG <-> FV projections of the listed cells (Limiter.cpp:23-112).

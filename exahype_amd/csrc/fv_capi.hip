@@ -2,6 +2,7 @@
 // FiniteVolumesSolver surface and a device-resident periodic patch grid.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstring>
 #include <mutex>
 #include <vector>
@@ -30,8 +31,8 @@ struct exa_fv_solver {
 };
 
 // MUSCL-Hancock kernel of a patch size (2..15 subcells per direction).
-using MusclFn = void (*)(const double*, double*, double*, unsigned long long*, PatchGeom, double, double, double,
-                         const double*, double, double);
+using MusclFn = void (*)(const double*, double*, double*, unsigned long long*, unsigned long long*, double, double,
+                         double, const double*, double, double, double);
 struct MusclLaunch {
   MusclFn fn;
   int threads;
@@ -100,22 +101,38 @@ static void patch_soa_to_ref(const double* soa, double* ref, int nbox) {
     for (int v = 0; v < FV_V; ++v) ref[c * FV_V + v] = soa[v * nbox + c];
 }
 
-// Launches the update of `np` patches: in -> out (out interior overwritten).
+static int subcells(const PatchGeom& g) { return g.dim == 3 ? g.P * g.P * g.P : g.P * g.P; }
+
+// The kernels that lay the patches' items end to end count them in 32 bits:
+// launch(first patch, patches, workgroups) over as many patches as that holds.
+template <class F>
+static void over_patches(int np, unsigned items, unsigned per_group, F launch) {
+  const int most = std::max(1, (int)((1u << 30) / items));
+  for (int p0 = 0; p0 < np; p0 += most) {
+    const int n = np - p0 < most ? np - p0 : most;
+    launch(p0, n, dim3(((unsigned)n * items + per_group - 1) / per_group));
+  }
+}
+
+// Launches the update of `np` patches (one, with dt_patch): in -> out (out interior overwritten);
+// the minima of the faces' and of the new states' CFL time steps go to the slots, or null.
 static int launch_fv_update(const exa_fv_solver* s, hipStream_t st, int np, const double* in, double* out,
-                            double* dt_patch, unsigned long long* dt_min, const double dx[3], const double* dt) {
+                            double* dt_patch, unsigned long long* adm_slots, unsigned long long* next_slots,
+                            const double dx[3], const double* dt) {
   const PatchGeom g = s->geom();
-  const double gam = s->cfg.gamma;
+  const double gam = s->cfg.gamma, cfl = s->cfg.cfl;
   if (s->cfg.scheme == EXA_FV_MUSCLHANCOCK) {
     // the kernel's own CFL (kernels/finitevolumes/musclhancock/c/musclhancock.h:29)
     const MusclLaunch m = muscl_kernel(g.P);
-    hipLaunchKernelGGL(m.fn, dim3(np), dim3(m.threads), m.lds, st, in, out, dt_patch, dt_min, g, dx[0], dx[1], dx[2],
-                       dt, gam, 0.99);
-  } else if (s->cfg.dim == 3) {
-    hipLaunchKernelGGL((exa::fv::k_godunov<3, EulerPDE>), dim3(np), dim3(256), 0, st, in, out, dt_patch, dt_min, g,
-                       dx[0], dx[1], dx[2], dt, gam, s->cfg.cfl);
+    hipLaunchKernelGGL(m.fn, dim3(np), dim3(m.threads), m.lds, st, in, out, dt_patch, adm_slots, next_slots, dx[0], dx[1],
+                       dx[2], dt, gam, 0.99, cfl);
   } else {
-    hipLaunchKernelGGL((exa::fv::k_godunov<2, EulerFV2DPDE>), dim3(np), dim3(256), 0, st, in, out, dt_patch, dt_min,
-                       g, dx[0], dx[1], dx[2], dt, gam, s->cfg.cfl);
+    const auto fn = s->cfg.dim == 3 ? &exa::fv::k_godunov<3, EulerPDE> : &exa::fv::k_godunov<2, EulerFV2DPDE>;
+    over_patches(np, subcells(g), 256, [&](int p0, int n, dim3 groups) {
+      // a patch's own minimum: one workgroup
+      hipLaunchKernelGGL(fn, dt_patch ? dim3(1) : groups, dim3(256), 0, st, in, out, dt_patch, adm_slots, next_slots, g,
+                         p0, n, dx[0], dx[1], dx[2], dt, gam, cfl);
+    });
   }
   EXA_CHECK(hipGetLastError());
   return EXA_OK;
@@ -149,7 +166,7 @@ extern "C" int exa_fv_solution_update(exa_fv_solver* s, double* luh_new, const d
   patch_ref_to_soa(luh_new, h.data(), nbox);
   EXA_CHECK(hipMemcpy(s->b.p, h.data(), sizeof(double) * h.size(), hipMemcpyHostToDevice));
   EXA_CHECK(hipMemcpy(s->st.as<double>() + 1, &dt, sizeof(double), hipMemcpyHostToDevice));
-  EXA_TRY(launch_fv_update(s, s->stream, 1, s->a.as<double>(), s->b.as<double>(), s->st.as<double>(), nullptr, dx,
+  EXA_TRY(launch_fv_update(s, s->stream, 1, s->a.as<double>(), s->b.as<double>(), s->st.as<double>(), nullptr, nullptr, dx,
                            s->st.as<double>() + 1));
   EXA_CHECK(hipStreamSynchronize(s->stream));
   EXA_CHECK(hipMemcpy(h.data(), s->b.p, sizeof(double) * h.size(), hipMemcpyDeviceToHost));
@@ -231,14 +248,21 @@ struct exa_fv_grid {
   double* dt_cur() const { return state.as<double>(); }
   unsigned long long* dt_next() const { return reinterpret_cast<unsigned long long*>(state.as<double>() + 1); }
   double* time() const { return state.as<double>() + 2; }
-  unsigned long long* adm() const { return reinterpret_cast<unsigned long long*>(state.as<double>() + 3); }
+  double* adm() const { return state.as<double>() + 3; }
+  // the admissible (0) and the next (1) time step of the step under way
+  unsigned long long* slots(int i) const {
+    return reinterpret_cast<unsigned long long*>(state.as<double>() + 8 + i * exa::fv::MIN_WORDS);
+  }
 };
 
-__global__ void k_fv_dt_advance(double* dt_cur, unsigned long long* dt_next, double* time) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
+// The step's minima out of their slots, and the clock: one wave.
+__global__ __launch_bounds__(64) void k_fv_dt_advance(double* dt_cur, double* adm, double* time,
+                                                      unsigned long long* adm_slots, unsigned long long* next_slots) {
+  const double a = exa::fv::take_minimum(adm_slots), n = exa::fv::take_minimum(next_slots);
+  if (threadIdx.x == 0) {
     *time += *dt_cur;
-    *dt_cur = __longlong_as_double((long long)*dt_next);
-    *dt_next = (unsigned long long)__double_as_longlong(1.0e300);
+    *dt_cur = n;
+    *adm = a;
   }
 }
 
@@ -389,16 +413,17 @@ extern "C" int exa_fv_grid_create(exa_fv_solver* s, int nx, int ny, int nz, cons
   int r = EXA_OK;
   if ((r = g->cur.ensure(sizeof(double) * psz * g->np)) != EXA_OK ||
       (r = g->nxt.ensure(sizeof(double) * psz * g->np)) != EXA_OK ||
-      (r = g->nbr.ensure(sizeof(int) * 6 * g->np)) != EXA_OK || (r = g->state.ensure(sizeof(double) * 8)) != EXA_OK) {
+      (r = g->nbr.ensure(sizeof(int) * 6 * g->np)) != EXA_OK || (r = g->state.ensure(sizeof(double) * (8 + 2 * exa::fv::MIN_WORDS))) != EXA_OK) {
     delete g;
     return r;
   }
   hipError_t e = fv_grid_neighbours(g);
-  double st[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  std::vector<double> st(8 + 2 * exa::fv::MIN_WORDS, 0.0);
   const unsigned long long bb = exa_big_bits();
   std::memcpy(&st[1], &bb, 8);
   std::memcpy(&st[3], &bb, 8);
-  if (e == hipSuccess) e = hipMemcpy(g->state.p, st, sizeof(st), hipMemcpyHostToDevice);
+  for (int i = 0; i < 2 * exa::fv::MIN_SLOTS; ++i) std::memcpy(&st[8 + i * exa::fv::MIN_STRIDE], &bb, 8);
+  if (e == hipSuccess) e = hipMemcpy(g->state.p, st.data(), sizeof(double) * st.size(), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemset(g->cur.p, 0, sizeof(double) * psz * g->np);
   if (e == hipSuccess) e = hipMemset(g->nxt.p, 0, sizeof(double) * psz * g->np);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking);
@@ -530,6 +555,8 @@ extern "C" int exa_fv_grid_step(exa_fv_grid* g, int nsteps) {
   fb.ny = g->ny;
   fb.time = g->time();
   fb.gamma = g->s->cfg.gamma;
+  const bool closed = !(g->periodic[0] && g->periodic[1] && g->periodic[2]);
+  const unsigned places = 2 * geo.dim * geo.G * (subcells(geo) / geo.P);
   for (int i = 0; i < nsteps; ++i) {
     hipEvent_t m[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
     if (g->timing) {
@@ -537,23 +564,25 @@ extern "C" int exa_fv_grid_step(exa_fv_grid* g, int nsteps) {
       g->marks.emplace_back(m, m + 5);
       EXA_CHECK(hipEventRecord(m[0], g->stream));
     }
-    if (g->s->cfg.dim == 3)
-      hipLaunchKernelGGL(exa::fv::k_fv_ghosts<3>, dim3(g->np), dim3(256), 0, g->stream, g->cur.as<double>(),
-                         g->nbr.as<int>(), geo, g->np, fb);
-    else
-      hipLaunchKernelGGL(exa::fv::k_fv_ghosts<2>, dim3(g->np), dim3(256), 0, g->stream, g->cur.as<double>(),
-                         g->nbr.as<int>(), geo, g->np, fb);
+    double* cur = g->cur.as<double>();
+    const bool d3 = geo.dim == 3;
+    over_patches(g->np, places, d3 ? 1024 : 256, [&](int p0, int n, dim3 groups) {
+      hipLaunchKernelGGL(d3 ? &exa::fv::k_fv_ghosts<3> : &exa::fv::k_fv_ghosts<2>, groups, dim3(256), 0, g->stream, cur,
+                         g->nbr.as<int>(), geo, g->np, p0, n);
+    });
+    if (closed)
+      hipLaunchKernelGGL(d3 ? &exa::fv::k_fv_boundary<3> : &exa::fv::k_fv_boundary<2>, dim3(g->np), dim3(256), 0,
+                         g->stream, cur, g->nbr.as<int>(), geo, g->np, fb);
     EXA_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(k_fv_reset, dim3(1), dim3(1), 0, g->stream, g->adm());
     if (m[1]) EXA_CHECK(hipEventRecord(m[1], g->stream));
     if (m[2]) EXA_CHECK(hipEventRecord(m[2], g->stream));  // phase 1 is empty (one update kernel)
-    EXA_TRY(launch_fv_update(g->s, g->stream, g->np, g->cur.as<double>(), g->nxt.as<double>(), nullptr, g->adm(),
-                             g->dx, g->dt_cur()));
+    EXA_TRY(launch_fv_update(g->s, g->stream, g->np, g->cur.as<double>(), g->nxt.as<double>(), nullptr, g->slots(0),
+                             g->slots(1), g->dx, g->dt_cur()));
     if (m[3]) EXA_CHECK(hipEventRecord(m[3], g->stream));
     g->cur.swap(g->nxt);
-    EXA_TRY(launch_fv_dt(g->s, g->stream, g->np, g->cur.as<double>(), nullptr, g->dt_next(), g->dx));
-    if (m[4]) EXA_CHECK(hipEventRecord(m[4], g->stream));
-    hipLaunchKernelGGL(k_fv_dt_advance, dim3(1), dim3(1), 0, g->stream, g->dt_cur(), g->dt_next(), g->time());
+    if (m[4]) EXA_CHECK(hipEventRecord(m[4], g->stream));  // the update's part of the time step included above
+    hipLaunchKernelGGL(k_fv_dt_advance, dim3(1), dim3(64), 0, g->stream, g->dt_cur(), g->adm(), g->time(),
+                       g->slots(0), g->slots(1));
     EXA_CHECK(hipGetLastError());
   }
   return EXA_OK;

@@ -58,98 +58,9 @@ __device__ inline int box_index(const PatchGeom& g, int i, int j, int k) {
   return g.dim == 3 ? (k * g.S + j) * g.S + i : j * g.S + i;
 }
 
-// The reference's face loops also run over the two patch-boundary faces of
-// every line, so the first ghost layer of luh_new receives one face update:
-// -= at the lower ghost (face ghost|first), += at the upper ghost (last|ghost).
-// Enumerates those cells: item -> (direction d, side, transverse position).
-__device__ inline void ghost_layer_cell(const PatchGeom& g, int item, int& d, int& side, int& idx, int& inner) {
-  const int trans = g.dim == 3 ? g.P * g.P : g.P;
-  d = item / (2 * trans);
-  side = (item / trans) % 2;
-  const int t = item % trans;
-  const int a = g.dim == 3 ? t / g.P + g.G : 0, b = t % g.P + g.G;
-  int c[3];
-  const int o1 = d == 0 ? 1 : 0, o2 = d == 2 ? 1 : 2;
-  c[o1] = b;
-  c[o2] = a;
-  c[d] = side ? g.G + g.P : g.G - 1;
-  idx = box_index(g, c[0], c[1], c[2]);
-  c[d] = side ? g.G + g.P - 1 : g.G;
-  inner = box_index(g, c[0], c[1], c[2]);
-}
-
-// Godunov update of every patch: luh_new(interior) = luh + flux differences.
-// Returns (per patch, and as a global minimum) the admissible dt of the face
-// wave speeds: min CFL/DIM * h / s_max (godunov.cpph:33-143).
-template <int DIM, class PDE>
-__global__ __launch_bounds__(256) void k_godunov(const double* __restrict__ luh, double* __restrict__ luh_new,
-                                                 double* __restrict__ dt_patch, unsigned long long* dt_min,
-                                                 PatchGeom g, double dx0, double dx1, double dx2,
-                                                 const double* __restrict__ dtp, double gamma, double cfl) {
-  __shared__ double red[8];
-  const double dt = *dtp;
-  const int nbox = g.ncells_box();
-  const double* u = luh + (size_t)blockIdx.x * V * nbox;
-  double* un = luh_new + (size_t)blockIdx.x * V * nbox;
-  const double h[3] = {dx0 / g.P, dx1 / g.P, dx2 / g.P};
-  const int ninterior = DIM == 3 ? g.P * g.P * g.P : g.P * g.P;
-  double dtm = 1.0e300;
-  for (int c = threadIdx.x; c < ninterior; c += blockDim.x) {
-    int i, j, k;
-    interior_coords(g, c, i, j, k);
-    const int idx = box_index(g, i, j, k);
-    double q[V], acc[V], qn[V], f[V];
-    load_q(u, nbox, idx, q);
-#pragma unroll
-    for (int v = 0; v < V; ++v) acc[v] = q[v];
-#pragma unroll
-    for (int d = 0; d < DIM; ++d) {
-      const double fac = dt / h[d];
-      load_q(u, nbox, idx - g.stride(d), qn);
-      double s = rusanov<PDE>(qn, q, d, gamma, f);
-      double cand = exa_dt_sane(cfl / DIM * h[d] / s);
-      dtm = cand < dtm ? cand : dtm;
-#pragma unroll
-      for (int v = 0; v < V; ++v) acc[v] += fac * f[v];
-      load_q(u, nbox, idx + g.stride(d), qn);
-      s = rusanov<PDE>(q, qn, d, gamma, f);
-      cand = exa_dt_sane(cfl / DIM * h[d] / s);
-      dtm = cand < dtm ? cand : dtm;
-#pragma unroll
-      for (int v = 0; v < V; ++v) acc[v] -= fac * f[v];
-    }
-#pragma unroll
-    for (int v = 0; v < V; ++v) un[v * nbox + idx] = acc[v];
-  }
-  const int nghost = 2 * DIM * (DIM == 3 ? g.P * g.P : g.P);
-  for (int it = threadIdx.x; it < nghost; it += blockDim.x) {
-    int d, side, idx, inner;
-    ghost_layer_cell(g, it, d, side, idx, inner);
-    double ql[V], qr[V], f[V];
-    load_q(u, nbox, side ? inner : idx, ql);
-    load_q(u, nbox, side ? idx : inner, qr);
-    rusanov<PDE>(ql, qr, d, gamma, f);
-    const double fac = dt / h[d];
-#pragma unroll
-    for (int v = 0; v < V; ++v) {
-      const double o = un[v * nbox + idx];
-      un[v * nbox + idx] = side ? o + fac * f[v] : o - fac * f[v];
-    }
-  }
-  dtm = block_min(dtm, red);
-  if (threadIdx.x == 0) {
-    if (dt_patch) dt_patch[blockIdx.x] = dtm;
-    if (dt_min) atomic_min_pos_double(dt_min, dtm);
-  }
-}
-
-__device__ inline double minmod(double a, double b) {
-  const double m = fabs(a) < fabs(b) ? a : b;
-  return a * b < 0.0 ? 0.0 : m;
-}
-
-// Admissible time step of faces with wave speeds s: the smallest exa_dt_sane(
-// cfl_h / s), with one division for the largest speed instead of one a face.
+// Admissible time step of faces (or subcells) with wave speeds s: the smallest
+// exa_dt_sane(cfl_h / s), with one division for the largest speed instead of
+// one a face.
 struct FaceSpeeds {
   double hi = 0.0;
   bool bad = false;
@@ -162,6 +73,114 @@ struct FaceSpeeds {
     return bad ? 0.0 : (hi > 0.0 ? exa_dt_sane(cfl_h / hi) : 1.0e300);
   }
 };
+
+// Wave speeds of a state in every direction, for the CFL time step (as k_fv_stable_dt).
+template <int DIM, class PDE>
+__device__ inline void add_state(FaceSpeeds* speeds, bool subcell, const double* q, const double* cfl_h, double gamma) {
+#pragma unroll
+  for (int d = 0; d < DIM; ++d) speeds[d].add(subcell, PDE::max_abs_eigenvalue(q, d, gamma), cfl_h[d]);
+}
+template <int DIM>
+__device__ inline double admissible(const FaceSpeeds* speeds, const double* cfl_h) {
+  double dtm = 1.0e300;
+#pragma unroll
+  for (int d = 0; d < DIM; ++d) {
+    const double cand = speeds[d].candidate(cfl_h[d]);
+    dtm = cand < dtm ? cand : dtm;
+  }
+  return dtm;
+}
+
+// A grid's minimum over its workgroups, kept in SLOTS words a cache line apart:
+// the workgroups that start together all find the word of a single minimum
+// still high and each take their turn at it, 12 ns one after the other (81 x 81
+// patches of 10^2, two minima: k_godunov 48.9 -> 45 us).
+constexpr int MIN_SLOTS = 64, MIN_STRIDE = 16;
+constexpr int MIN_WORDS = MIN_SLOTS * MIN_STRIDE;
+
+// The workgroup's smallest value: as its patch's, and into the grid's slots.
+__device__ inline void put_minimum(double v, double* red, double* dt_patch, unsigned long long* slots) {
+  v = block_min(v, red);
+  if (threadIdx.x == 0) {
+    if (dt_patch) dt_patch[blockIdx.x] = v;
+    if (slots) atomic_min_pos_double(slots + blockIdx.x % MIN_SLOTS * MIN_STRIDE, v);
+  }
+}
+
+// One wave: the slots' minimum, and the slots cleared for the next step.
+__device__ inline double take_minimum(unsigned long long* slots) {
+  unsigned long long* w = slots + threadIdx.x % MIN_SLOTS * MIN_STRIDE;
+  const double v = __longlong_as_double((long long)*w);
+  *w = (unsigned long long)__double_as_longlong(1.0e300);
+  return wave_min(v);
+}
+
+// Godunov update of patches p0 .. p0 + np - 1: luh_new(interior) = luh + flux
+// differences, and the patch-boundary face updates of the first ghost layer by
+// the subcells beside it, which have just formed those fluxes (the reference's
+// face loops run over both patch-boundary faces of every line: -= at the lower
+// ghost, += at the upper one).  Also the admissible dt of the face wave speeds,
+// min CFL/DIM * h / s_max (godunov.cpph:33-143), as a global minimum or, one
+// patch in one workgroup, in dt_patch; next_slots: the CFL time step of the new
+// states too (null: not asked for), which are at hand here.
+// One subcell a thread, the patches' subcells end to end: a 10^2 patch fills 39
+// of 100 lanes of a workgroup of its own.  Bound by the latency of its loads;
+// 81 x 81 patches of 10^2: 45 us, with a workgroup a patch, the ghost
+// layers' fluxes formed again and a pass of its own for the time step 72.
+template <int DIM, class PDE>
+__global__ __launch_bounds__(256) void k_godunov(const double* __restrict__ luh, double* __restrict__ luh_new,
+                                                 double* __restrict__ dt_patch, unsigned long long* adm_slots,
+                                                 unsigned long long* next_slots, PatchGeom g, int p0, int np, double dx0,
+                                                 double dx1, double dx2, const double* __restrict__ dtp, double gamma,
+                                                 double cfl) {
+  __shared__ double red[8];
+  const double dt = *dtp;
+  const int nbox = g.ncells_box();
+  const double h[3] = {dx0 / g.P, dx1 / g.P, dx2 / g.P};
+  const unsigned ninterior = DIM == 3 ? g.P * g.P * g.P : g.P * g.P;
+  const double cfl_h[3] = {cfl / DIM * h[0], cfl / DIM * h[1], cfl / DIM * h[2]};
+  FaceSpeeds speeds[DIM], next[DIM];
+  for (unsigned it = blockIdx.x * blockDim.x + threadIdx.x; it < np * ninterior; it += gridDim.x * blockDim.x) {
+    const double* u = luh + (size_t)(p0 + it / ninterior) * V * nbox;
+    double* un = luh_new + (size_t)(p0 + it / ninterior) * V * nbox;
+    int ijk[3];
+    interior_coords(g, it % ninterior, ijk[0], ijk[1], ijk[2]);
+    const int idx = box_index(g, ijk[0], ijk[1], ijk[2]);
+    double q[V], acc[V], qn[V], f[V];
+    load_q(u, nbox, idx, q);
+#pragma unroll
+    for (int v = 0; v < V; ++v) acc[v] = q[v];
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) {
+      const double fac = dt / h[d];
+      const int o = g.stride(d);
+      load_q(u, nbox, idx - o, qn);
+      speeds[d].add(true, rusanov<PDE>(qn, q, d, gamma, f), cfl_h[d]);
+#pragma unroll
+      for (int v = 0; v < V; ++v) acc[v] += fac * f[v];
+      if (ijk[d] == g.G)
+#pragma unroll
+        for (int v = 0; v < V; ++v) un[v * nbox + idx - o] = un[v * nbox + idx - o] - fac * f[v];
+      load_q(u, nbox, idx + o, qn);
+      speeds[d].add(true, rusanov<PDE>(q, qn, d, gamma, f), cfl_h[d]);
+#pragma unroll
+      for (int v = 0; v < V; ++v) acc[v] -= fac * f[v];
+      if (ijk[d] == g.G + g.P - 1)
+#pragma unroll
+        for (int v = 0; v < V; ++v) un[v * nbox + idx + o] = un[v * nbox + idx + o] + fac * f[v];
+    }
+#pragma unroll
+    for (int v = 0; v < V; ++v) un[v * nbox + idx] = acc[v];
+    if (next_slots) add_state<DIM, PDE>(next, true, acc, cfl_h, gamma);
+  }
+  put_minimum(admissible<DIM>(speeds, cfl_h), red, dt_patch, adm_slots);
+  if (next_slots) put_minimum(admissible<DIM>(next, cfl_h), red, nullptr, next_slots);
+}
+
+__device__ inline double minmod(double a, double b) {
+  const double m = fabs(a) < fabs(b) ? a : b;
+  return a * b < 0.0 ? 0.0 : m;
+}
 
 // A value is formed here, and not at its first use.
 __device__ inline void fv_pin(double& x) { asm volatile("" : "+v"(x)); }
@@ -191,7 +210,8 @@ __device__ inline double wave_uniform(double x) {
 // cover each other's waits, if 168 registers hold a thread: values that wait
 // longest stay in the LDS or are loaded again, since a spilled register's
 // reload also waits for every load in flight (24 spills: 344 us).
-// 12 x 13 x 14 patches of 11^3: 232 us.  Forming the states of each subcell
+// 12 x 13 x 14 patches of 11^3: 232 us, 258 with the new states' time step (a
+// pass of its own: 41).  Forming the states of each subcell
 // and face where they are used, every state four times: 527; one thread per
 // two subcells, a patch's states in the LDS at once, one workgroup per compute
 // unit: 400.
@@ -204,11 +224,11 @@ struct MusclForm {
 
 // One patch: u (with its ghost layers) -> un (interior and the first ghost
 // layer's face updates); sm: MusclForm<PC>::LDS bytes.  Returns the thread's
-// part of the admissible time step.
-template <class PDE, int PC>
+// part of the admissible time step; NEXT: adds the new states' speeds to next[3].
+template <class PDE, int PC, bool NEXT>
 __device__ __forceinline__ double muscl_patch(const double* __restrict__ u, double* __restrict__ un, double* sm,
                                               double dx0, double dx1, double dx2, double dt, double gamma,
-                                              double cfl) {
+                                              double cfl, FaceSpeeds* next = nullptr, const double* next_h = nullptr) {
   constexpr int S = PC + 4, T = PC + 2, PL = S * S, nbox = S * PL, TT = T * T;
   const double h[3] = {dx0 / PC, dx1 / PC, dx2 / PC};
   const double fac[3] = {wave_uniform(dt / h[0]), wave_uniform(dt / h[1]), wave_uniform(dt / h[2])};
@@ -350,6 +370,7 @@ __device__ __forceinline__ double muscl_patch(const double* __restrict__ u, doub
     }
     z_face(w, f);
     if (z > 2 ? kept : inner) store_node(z - 1, acc);
+    if (NEXT) add_state<3, PDE>(next, inner && z > 2, acc, next_h, gamma);
 #pragma unroll
     for (int v = 0; v < V; ++v) wz[v] = hs[2][v];
     __builtin_amdgcn_sched_barrier(0);
@@ -397,36 +418,33 @@ __device__ __forceinline__ double muscl_patch(const double* __restrict__ u, doub
   for (int v = 0; v < V; ++v) w[v] = q[v] - 0.5 * minmod(qp[v] - q[v], q[v] - qm[v]);
   z_face(w, f);
   if (kept) store_node(PC + 1, acc);
+  if (NEXT) add_state<3, PDE>(next, inner, acc, next_h, gamma);
   if (inner) {
     load_node(un, PC + 2, col, acc);
 #pragma unroll
     for (int v = 0; v < V; ++v) acc[v] += f[v];
     store_node(PC + 2, acc);
   }
-  double dtm = 1.0e300;
-#pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    const double cand = speeds[d].candidate(cfl_h[d]);
-    dtm = cand < dtm ? cand : dtm;
-  }
-  return dtm;
+  return admissible<3>(speeds, cfl_h);
 }
 
+// next_slots: the CFL time step (factor next_cfl) of the new states, or null.
 template <class PDE, int PC>
 __global__ __launch_bounds__(MusclForm<PC>::NT) __attribute__((amdgpu_waves_per_eu(3))) void k_muscl(
     const double* __restrict__ luh, double* __restrict__ luh_new, double* __restrict__ dt_patch,
-    unsigned long long* dt_min, PatchGeom, double dx0, double dx1, double dx2, const double* __restrict__ dtp,
-    double gamma, double cfl) {
+    unsigned long long* adm_slots, unsigned long long* next_slots, double dx0, double dx1, double dx2,
+    const double* __restrict__ dtp, double gamma, double cfl, double next_cfl) {
   extern __shared__ double sm[];
-  __shared__ double red[16];
+  __shared__ double red[8];
   constexpr int nbox = (PC + 4) * (PC + 4) * (PC + 4);
-  double dtm = muscl_patch<PDE, PC>(luh + (size_t)blockIdx.x * V * nbox, luh_new + (size_t)blockIdx.x * V * nbox, sm,
-                                  dx0, dx1, dx2, *dtp, gamma, cfl);
-  dtm = block_min(dtm, red);
-  if (threadIdx.x == 0) {
-    if (dt_patch) dt_patch[blockIdx.x] = dtm;
-    if (dt_min) atomic_min_pos_double(dt_min, dtm);
-  }
+  const double next_h[3] = {wave_uniform(next_cfl / 3 * (dx0 / PC)), wave_uniform(next_cfl / 3 * (dx1 / PC)),
+                            wave_uniform(next_cfl / 3 * (dx2 / PC))};
+  FaceSpeeds next[3];
+  const double dtm =
+      muscl_patch<PDE, PC, true>(luh + (size_t)blockIdx.x * V * nbox, luh_new + (size_t)blockIdx.x * V * nbox, sm, dx0,
+                                 dx1, dx2, *dtp, gamma, cfl, next, next_h);
+  put_minimum(dtm, red, dt_patch, adm_slots);
+  if (next_slots) put_minimum(admissible<3>(next, next_h), red, nullptr, next_slots);
 }
 
 // FV CFL time step of every patch (commons.cpph:26-67 2D, :410-463 3D).
@@ -523,41 +541,77 @@ struct FvBoundary {
   double gamma;
 };
 
-// Face ghost layers: from the neighbours' interiors (ghostLayerFilling,
-// commons.cpph:337-402, :876-982), or, where a closed axis leaves no
-// neighbour (nbr < 0), as mergeWithBoundaryData fills them
-// (E/solvers/FiniteVolumesSolver.cpp:689-728): the mirrored layer of the
-// boundary-layer extraction through boundaryValues.  nbr[(2*d + side)*npatch
-// + p]: neighbour of patch p on side (0: -, 1: +) of direction d.
+// Layer kk and transverse place t of a face's item; on the x faces the layers
+// come first: they lie beside each other in memory.
+__device__ inline void fv_ghost_place(const PatchGeom& g, int trans, int d, int r, int& kk, int& t) {
+  kk = d == 0 ? r % g.G : r / trans;
+  t = d == 0 ? r / g.G : r % trans;
+}
+
+// Face ghost layers of patches p0 .. p0 + np - 1 from the neighbours' interiors
+// (ghostLayerFilling, commons.cpph:337-402, :876-982).  nbr[(2*d + side)*npatch
+// + p]: neighbour of patch p on side (0: -, 1: +) of direction d, < 0 where a
+// closed axis leaves none.
+// The patches' places end to end, B of them a thread with all their loads in
+// flight before the first store.  Bound by memory lines in 3D: the x layers
+// touch most lines of a patch and of its x neighbours for two values each
+// (12 x 13 x 14 patches of 11^3: 119 us, 840 MB of lines), by launch and
+// latency in 2D (81 x 81 patches of 10^2: 19 us).
 template <int DIM>
-__global__ __launch_bounds__(256) void k_fv_ghosts(double* __restrict__ luh, const int* __restrict__ nbr,
-                                                   PatchGeom g, int npatch, FvBoundary fb) {
+__global__ __launch_bounds__(256) void k_fv_ghosts(double* __restrict__ luh, const int* __restrict__ nbr, PatchGeom g,
+                                                   int npatch, int p0, int np) {
+  constexpr int B = DIM == 3 ? 4 : 1;
+  const int nbox = g.ncells_box();
+  const int trans = DIM == 3 ? g.P * g.P : g.P;
+  const unsigned per_side = g.G * trans, total = 2 * DIM * per_side;
+  double w[B][V];
+  double* dst[B];
+#pragma unroll
+  for (int b = 0; b < B; ++b) {
+    const unsigned it = (blockIdx.x * B + b) * 256 + threadIdx.x, i = it < np * total ? it : 0;
+    const int p = p0 + i / total, ds = i % total / per_side, d = ds / 2, side = ds % 2;
+    int kk, t, o1, o2, c[3];
+    fv_ghost_place(g, trans, d, i % per_side, kk, t);
+    fv_axes(DIM, d, o1, o2);
+    c[o1] = t % g.P + g.G;
+    c[o2] = DIM == 3 ? t / g.P + g.G : 0;
+    c[d] = side ? g.G + g.P + kk : kk;
+    const int q = nbr[ds * npatch + p];
+    dst[b] = it < np * total && q >= 0 ? luh + (size_t)p * V * nbox + box_index(g, c[0], c[1], c[2]) : nullptr;
+    c[d] = side ? g.G + kk : g.P + kk;
+    load_q(luh + (size_t)(q >= 0 ? q : p) * V * nbox, nbox, box_index(g, c[0], c[1], c[2]), w[b]);
+  }
+#pragma unroll
+  for (int b = 0; b < B; ++b)
+    if (dst[b]) {
+#pragma unroll
+      for (int v = 0; v < V; ++v) dst[b][v * nbox] = w[b][v];
+    }
+}
+
+// Those without a neighbour, as mergeWithBoundaryData fills them
+// (E/solvers/FiniteVolumesSolver.cpp:689-728): the mirrored layer of the
+// boundary-layer extraction through boundaryValues.  One workgroup per patch,
+// launched where an axis is closed; kept apart because the analytical boundary
+// values take 130 registers.
+template <int DIM>
+__global__ __launch_bounds__(256) void k_fv_boundary(double* __restrict__ luh, const int* __restrict__ nbr,
+                                                     PatchGeom g, int npatch, FvBoundary fb) {
   const int p = blockIdx.x;
   const int nbox = g.ncells_box();
   const int trans = DIM == 3 ? g.P * g.P : g.P;
-  const int per_side = g.G * trans;
-  const int total = 2 * DIM * per_side;
   double* me = luh + (size_t)p * V * nbox;
-  for (int it = threadIdx.x; it < total; it += blockDim.x) {
-    const int ds = it / per_side, r = it % per_side;
+  for (int ds = 0; ds < 2 * DIM; ++ds) {
+    if (nbr[ds * npatch + p] >= 0) continue;
     const int d = ds / 2, side = ds % 2;
-    const int kk = r / trans, t = r % trans;
-    const int ta = DIM == 3 ? t / g.P : 0, tb = t % g.P;  // transverse interior indices
-    int o1, o2;
-    fv_axes(DIM, d, o1, o2);
-    int ci[3], ni[3];
-    ci[o1] = ni[o1] = tb + g.G;
-    ci[o2] = ni[o2] = DIM == 3 ? ta + g.G : 0;
-    ci[d] = side ? g.G + g.P + kk : kk;
-    const int q = nbr[(2 * d + side) * npatch + p];
-    if (q >= 0) {
-      ni[d] = side ? g.G + kk : g.P + kk;
-      const double* nb = luh + (size_t)q * V * nbox;
-      const int cidx = box_index(g, ci[0], ci[1], ci[2]);
-      const int nidx = box_index(g, ni[0], ni[1], ni[2]);
-#pragma unroll
-      for (int v = 0; v < V; ++v) me[v * nbox + cidx] = nb[v * nbox + nidx];
-    } else {
+    for (int r = threadIdx.x; r < g.G * trans; r += blockDim.x) {
+      int kk, t, o1, o2, ci[3], ni[3];
+      fv_ghost_place(g, trans, d, r, kk, t);
+      const int ta = DIM == 3 ? t / g.P : 0, tb = t % g.P;  // transverse interior indices
+      fv_axes(DIM, d, o1, o2);
+      ci[o1] = ni[o1] = tb + g.G;
+      ci[o2] = ni[o2] = DIM == 3 ? ta + g.G : 0;
+      ci[d] = side ? g.G + g.P + kk : kk;
       const int K = g.G - kk - 1;
       ni[d] = fv_extract_layer(DIM, d, side, g.P, g.G, K);
       const int px = p % fb.nx, py = (p / fb.nx) % fb.ny, pz = p / (fb.nx * fb.ny);

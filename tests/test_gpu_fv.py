@@ -128,3 +128,26 @@ def test_fv_grid_steps_vs_oracle(dim, patch, scheme, opde, n, steps):
     assert abs(dt_g - dt_o) <= 1e-12 * dt_o
     assert abs(adm_g - adm_o) <= 1e-12 * adm_o
     assert rel_err(interior(g.download()), interior(og.luh())) <= TOL
+
+
+@pytest.mark.parametrize("dim,patch,scheme,cells", [(2, 3, 0, (5, 3, 1)), (2, 10, 0, (7, 9, 1)), (2, 16, 0, (1, 1, 1)),
+                                                    (3, 4, 0, (3, 2, 5)), (3, 7, 0, (2, 3, 1)), (3, 5, 1, (9, 8, 3)),
+                                                    (3, 11, 1, (1, 2, 1))])
+def test_step_minima_are_those_of_the_separate_kernel(dim, patch, scheme, cells):
+    """The time step that the update leaves behind is the one the state itself
+    gives, to the bit, and the admissible one is no single patch's old value;
+    patches whose subcells do not fill workgroups, fewer and more workgroups
+    than there are words for the minima."""
+    import exahype_amd as E
+    s = E.FiniteVolumesSolver(dim, patch, scheme)
+    g = E.FVGrid(s, *cells)
+    rng = np.random.default_rng(patch)
+    g.upload(euler_state(rng, int(np.prod(cells)) * s.side ** dim))
+    g.compute_dt()
+    seen = []
+    for n in (1, 3):
+        g.step(n)
+        _, dt, adm = g.sync()
+        seen.append(adm)
+        assert dt == g.compute_dt() and 0 < dt < 1 and 0 < adm < 1
+    assert seen[0] != seen[1]
