@@ -46,7 +46,9 @@ __global__ __launch_bounds__(Ord<N>::NT) void k_predictor_pde(
   const int z = act ? s / B2 : 0, y = act ? (s / B) % B : 0, x = act ? s % B : 0;
   const double dt = *dtp;
   const double w3 = (T.w[z] * T.w[y]) * T.w[x];
-  const double iweight = 1.0 / w3;
+  const double idx0 = 1.0 / dx0, idx1 = 1.0 / dx1, idx2 = 1.0 / dx2;
+  // dt / dx over the node's own weight: the right-hand side times w^-3
+  const double sx = dt * idx0 / T.w[x], sy = dt * idx1 / T.w[y], sz = dt * idx2 / T.w[z];
 
   double u0[V], q[B][V];
 #pragma unroll
@@ -61,6 +63,13 @@ __global__ __launch_bounds__(Ord<N>::NT) void k_predictor_pde(
   int it = 0;
   for (int iter = 0; iter < MaxIterations; ++iter) {
     ++it;
+    // Every time node of the first iterate holds the state itself: one slice
+    // does for all B of them, since sum_t F0[t] iK1[l][t] = 1 (a constant
+    // solution) and sum_t w[t] iK1[l][t] = xi[l] (one that grows like time,
+    // which every order reproduces).  Advection through the non-conservative
+    // product, N = 4, 25 x 26 x 27 cells: 583 -> 454 us, with the weights'
+    // quotients and 1 / dx formed once.
+    const bool first = !DEBUG && iter == 0;
     double qn[B][V];
 #pragma unroll
     for (int t = 0; t < B; ++t)
@@ -74,6 +83,7 @@ __global__ __launch_bounds__(Ord<N>::NT) void k_predictor_pde(
     }
 #pragma unroll
     for (int t = 0; t < B; ++t) {
+      const double wt = t == 0 && first ? 1.0 : T.w[t];
       __syncthreads();  // the previous slice is consumed
       if (act) {
         if (PDE::NCP) {
@@ -88,7 +98,7 @@ __global__ __launch_bounds__(Ord<N>::NT) void k_predictor_pde(
 #pragma unroll
             for (int v = 0; v < V; ++v) {
               sF[(d * V + v) * B3 + s] = F[d][v];
-              fh[d][v] += F[d][v] * T.w[t];  // time average of the sweep (:326-397)
+              fh[d][v] += F[d][v] * wt;  // time average of the sweep (:326-397)
             }
         }
         if (DEBUG) {
@@ -126,7 +136,7 @@ __global__ __launch_bounds__(Ord<N>::NT) void k_predictor_pde(
           const int d = k / (V * B2), v = (k / B2) % V, ab = k % B2, a = ab / B, b = ab % B;
           const int base = d == 0 ? a * B2 + b * B : (d == 1 ? a * B2 + b : a * B + b);
           const int step = d == 0 ? 1 : (d == 1 ? B : B2);
-          const double idx = d == 0 ? 1.0 / dx0 : (d == 1 ? 1.0 / dx1 : 1.0 / dx2);
+          const double idx = d == 0 ? idx0 : (d == 1 ? idx1 : idx2);
           double pq[B];
 #pragma unroll
           for (int n = 0; n < B; ++n) pq[n] = sQ[v * B3 + base + n * step];
@@ -134,27 +144,22 @@ __global__ __launch_bounds__(Ord<N>::NT) void k_predictor_pde(
           for (int l = 0; l < B; ++l) {
             double g = 0.0;
 #pragma unroll
-            for (int n = 0; n < B; ++n) g += idx * pq[n] * T.dudx[l][n];
-            sG[(d * V + v) * B3 + base + l * step] = g;
+            for (int n = 0; n < B; ++n) g += pq[n] * T.dudx[l][n];
+            sG[(d * V + v) * B3 + base + l * step] = idx * g;
           }
         }
       }
       if (PDE::FLUX || PDE::NCP) __syncthreads();
       if (act) {
-        // rhs0 = w^3 F0 luh (:118-133)
+        // r: w^-3 (rhs - rhs0) (:136-252)
         double r[V];
-        const double c0 = w3 * T.F0[t];
 #pragma unroll
-        for (int v = 0; v < V; ++v) r[v] = c0 * u0[v];
-        if (PDE::FLUX) {  // rhs -= (w dt/dx) lFi Kxi per direction (:143-222)
-          const double usx = ((T.w[t] * T.w[z]) * T.w[y]) * dt / dx0;
-          const double usy = ((T.w[t] * T.w[z]) * T.w[x]) * dt / dx1;
-          const double usz = ((T.w[t] * T.w[y]) * T.w[x]) * dt / dx2;
-#pragma unroll
-          for (int v = 0; v < V; ++v) {
-            r[v] -= usx * sF[(0 * V + v) * B3 + s];
-            r[v] -= usy * sF[(1 * V + v) * B3 + s];
-            r[v] -= usz * sF[(2 * V + v) * B3 + s];
+        for (int v = 0; v < V; ++v) {
+          r[v] = 0.0;
+          if (PDE::FLUX) {  // - (w dt/dx) lFi Kxi per direction (:143-222)
+            r[v] -= wt * sx * sF[(0 * V + v) * B3 + s];
+            r[v] -= wt * sy * sF[(1 * V + v) * B3 + s];
+            r[v] -= wt * sz * sF[(2 * V + v) * B3 + s];
           }
         }
         if (PDE::SRC || PDE::NCP) {
@@ -170,11 +175,10 @@ __global__ __launch_bounds__(Ord<N>::NT) void k_predictor_pde(
           }
           double S[V];
           fused_source<PDE>(q[t], G, S, P);
-          const double us = (((T.w[t] * T.w[z]) * T.w[y]) * T.w[x]) * dt;
 #pragma unroll
           for (int v = 0; v < V; ++v) {
-            r[v] += us * S[v];
-            sh[v] += S[v] * T.w[t];
+            r[v] += wt * dt * S[v];
+            sh[v] += S[v] * wt;
           }
           if (DEBUG) {
 #pragma unroll
@@ -184,12 +188,25 @@ __global__ __launch_bounds__(Ord<N>::NT) void k_predictor_pde(
 #pragma unroll
           for (int v = 0; v < V; ++v) dbg.lFi[((t * B3 + s) * 4 + 3) * V + v] = 0.0;
         }
-        // this time node's share of the new iterate: += (w^-3 rhs) iK1 (:270-296)
+        if (t == 0 && first) {
 #pragma unroll
-        for (int l = 0; l < B; ++l)
+          for (int l = 0; l < B; ++l)
 #pragma unroll
-          for (int v = 0; v < V; ++v) qn[l][v] += iweight * r[v] * T.iK1[l][t];
+            for (int v = 0; v < V; ++v) qn[l][v] = u0[v] + T.xi[l] * r[v];
+        } else {
+          // rhs0 = w^3 F0 luh (:118-133), and this time node's share of the new
+          // iterate: += (w^-3 rhs) iK1 (:270-296)
+#pragma unroll
+          for (int v = 0; v < V; ++v) r[v] += T.F0[t] * u0[v];
+#pragma unroll
+          for (int l = 0; l < B; ++l)
+#pragma unroll
+            for (int v = 0; v < V; ++v) {
+              qn[l][v] += r[v] * T.iK1[l][t];
+            }
+        }
       }
+      if (t == 0 && first) break;
     }
     // exit condition (:299-306)
     double res = 0.0;

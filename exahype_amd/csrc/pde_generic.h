@@ -159,11 +159,12 @@ struct PdeEulerNcpTest {
 // kernels::fusedSource (kernels/fusedMethods.cpph:17-32): S = algebraicSource
 // (or 0) minus the non-conservative product.
 template <class PDE>
-__device__ inline void fused_source(const double* Q, const double G[3][5], double S[5], const PdeParams& p) {
+__device__ __forceinline__ void fused_source(const double* Q, const double G[3][5], double S[5], const PdeParams& p) {
   PDE::source(Q, S, p);
   if (PDE::NCP) {
     double n[5];
     PDE::ncp(Q, G, n, p);
+#pragma unroll
     for (int v = 0; v < 5; ++v) S[v] -= n[v];
   }
 }

@@ -146,6 +146,27 @@ def test_grid_steps_vs_oracle(pde, N, dims, steps):
     assert rel_err(g.download(), og.luh()) <= TOL
 
 
+@pytest.mark.parametrize("pde", [3, 4, 5])
+@pytest.mark.parametrize("N", [1, 2, 4, 6])
+def test_first_sweep_from_one_slice(pde, N):
+    """The orders that the test above leaves out: the iterate after the first
+    sweep, which steps form from one time node's terms, against the oracle's
+    loop over all of them -- the same bar and sweep counts, also for a state
+    at rest, where the first sweep is the last but one and its averages count."""
+    g, og = _grid_pair(pde, N, (3, 2, 2), _vortex_ic() if pde == 5 else _sine_ic())
+    for uniform in (False, True):
+        if uniform and pde != 5:
+            og.luh()[:] = np.tile([1.0, 0.3, -0.2, 0.1, 2.5], og.luh().size // 5)
+            g.upload(og.luh().copy())
+        dt_o = og.stable_dt()
+        g.compute_dt()
+        g.step(1)
+        og.step(dt_o)
+        g.sync()
+        assert np.array_equal(g.picard_iterations(), og.iters())
+        assert rel_err(g.download(), og.luh()) <= TOL
+
+
 def test_negative_pressure_of_the_test_product_is_reported():
     """Euler with the reference test's product at N=7 on 2^3 cells: after two
     steps a node holds a negative pressure (the oracle's state, below), where
