@@ -33,6 +33,24 @@ def _state(N, seed):
     return q.ravel()
 
 
+@pytest.mark.parametrize("gravity", [None, 9.81])
+@pytest.mark.parametrize("N", range(5, 10))
+def test_staged_first_sweep_vs_oracle(N, gravity):
+    """The staged form's one-slice first sweep: a cell that takes several, one
+    that stops after it (its averages are then the first iterate's), and the
+    gravity source, whose share of the slice carries a weight of its own."""
+    import exahype_amd as E
+    s = E.ADERDGSolver(N, contraction=E.CONTRACT_STAGED, gravity=gravity)
+    c = O.cfg(N) if gravity is None else O.cfg(N, pde=3, grav=gravity)
+    for seed, dx in ((1, np.array([1 / 27, 1 / 9, 1 / 20])), (None, np.array([0.1, 0.2, 0.3]))):
+        luh = _state(N, seed)
+        dt = 0.9 * O.stable_time_step_size(c, luh, dx)
+        g, o = s.spaceTimePredictor(luh, dx, dt), O.space_time_predictor(c, luh, dx, dt)
+        assert g["iters"] == o["iters"] and (seed is not None or gravity is not None or g["iters"] == 1)
+        for k in ("lQi", "lQhi", "lFhi", "lQhbnd", "lFhbnd"):
+            assert rel(g[k], o[k]) <= TOL, k
+
+
 @pytest.mark.parametrize("N", range(1, 9))
 def test_deferred_predictions_vs_oracle(N):
     import exahype_amd as E
