@@ -275,7 +275,7 @@ def main():
     ref50 = state_after(N, n, ERROR_STEPS, E.PREC_FP64, args.waves_per_simd, args.contraction)
     mixed = {}
     for name, prec, sweeps in MIXED_VARIANTS:
-        if N > 7 and prec != E.PREC_FP32:  # orders 8 and 9: FP32 sweeps on the staged predictor only
+        if N > 7 and prec != E.PREC_FP32:  # orders 8 and 9 have no matrix-core forms
             continue
         # the staged form takes FP64 and FP32 sweeps; the matrix-core forms their tuned form
         cm = 0 if (args.contraction == 4 and prec != E.PREC_FP32) else args.contraction
@@ -312,7 +312,9 @@ def main():
         flops = f_lp + f64
         peak_lp = PEAK_BF16_TFLOPS if best["prec"] == E.PREC_BF16_MFMA else PEAK_FP32_TFLOPS
         peak = flops / (f_lp / peak_lp + f64 / PEAK_FP64_TFLOPS)
-        kname = "k_predictor<%d, %s + %d FP64 sweep(s)>" % (N, best["name"], best["sweeps_fp64"])
+        hist = best["prec"] == E.PREC_FP32 and args.contraction == 0 and args.waves_per_simd == 0 and N <= 8
+        kname = "k_predictor%s<%d, %s + %d FP64 sweep(s)>" % ("_history" if hist else "", N, best["name"],
+                                                              best["sweeps_fp64"])
         # what bounds each part: FP32 sweeps on the vector ALU (no packed
         # FP32), MFMA forms on the matrix cores, FP64 sweeps and tail on the
         # FP64 vector ALU
@@ -321,7 +323,8 @@ def main():
     else:
         flops = predictor_flops_per_cell(N, sweeps) * ncells
         peak = PEAK_FP64_TFLOPS
-        kname = "k_predictor<%d, FP64>" % N
+        hist = args.contraction == 0 and args.waves_per_simd == 0 and N <= 8
+        kname = "k_predictor%s<%d, FP64>" % ("_history" if hist else "", N)
         bound = "fp64_valu"
     achieved = flops / (pred_ms * 1e-3) / 1e12
 
@@ -1061,7 +1064,7 @@ def run_amr_limiter(args):
                       "parallelism": "single GPU"},
            "precisions": runs,
            "roofline": {"bound": "fp32_valu+fp64", "achieved": achieved, "peak": peak, "unit": "TFLOP/s",
-                        "frac": achieved / peak, "traffic": None, "kernel": "k_predictor<5, fp32 + 1 FP64 sweep>",
+                        "frac": achieved / peak, "traffic": None, "kernel": "k_predictor_history<5, fp32 + 1 FP64 sweep>",
                         "avg_launch_ms": pred_ms, "picard_sweeps_per_cell_step": sw, "flop_per_launch": flop},
            "timing": "value: wall clock of the steps replayed as one hipGraph per step; phase_ms_per_step: HIP "
                      "events around the stages of 3 further steps (graph off)"}

@@ -266,9 +266,10 @@ struct TunedVariant {
 };
 static TunedVariant g_tuned[64][EXA_MAX_ORDER + 1][4];
 
-// The staged predictor: orders 8, 9, chosen explicitly, or the measured
-// default of the FP64 predictor at N = 7 (81^3 cells: 222 ms per launch
-// staged vs 339 ms register-resident, whose sweeps spill at that order).
+// The staged predictor: orders 8, 9, chosen explicitly, or at N = 7 in FP64
+// where predictor_history does not serve (the gravity source, per-cell
+// outputs; 81^3 cells: 222 ms per launch staged vs 339 ms register-resident,
+// whose sweeps spill at that order).  Callers ask predictor_history first.
 static bool predictor_staged(const exa_aderdg_config& c, int dev) {
   if (exa_pde_generic(c.pde)) return false;
   if (c.order >= 8 || c.contraction == EXA_CONTRACT_STAGED) return true;
@@ -280,7 +281,7 @@ static bool predictor_staged(const exa_aderdg_config& c, int dev) {
 // (pred_history.hip; faster than every other form at orders 1..8, see
 // aderdg_history.h), unless the configuration or exa_autotune asks for another
 // form.  At order 9 its registers do not hold
-// the state (7.8 ms against the staged form's 6.8 at 18^3 cells, FP64).
+// the state (7.8 ms against the staged form's 5.7 at 18^3 cells, FP64).
 static bool predictor_history(const exa_aderdg_config& c, int dev) {
   return c.pde == EXA_PDE_EULER && !c.linear && c.order >= EXA_HISTORY_MIN_ORDER &&
          c.order <= EXA_HISTORY_MAX_ORDER &&

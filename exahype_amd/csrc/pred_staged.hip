@@ -1,5 +1,6 @@
 // Predictor kernels with the space-time iterate staged in global memory:
-// the only form of orders 8 and 9, selectable (EXA_CONTRACT_STAGED) at 5..7;
+// the form of order 9 (and of per-cell outputs at order 8), selectable
+// (EXA_CONTRACT_STAGED) at 5..8;
 // FP64, FP64 with the gravity source, and mixed (an FP32 phase).
 #include "aderdg_kernels.h"
 #include "predictor_tu.h"

@@ -152,8 +152,8 @@ typedef struct {
 #define EXA_CONTRACT_PENCIL_PAIR 3 /* pencil owners, two slices per phase, contraction in place */
 #define EXA_CONTRACT_STAGED 4   /* space-time iterate staged in global memory (FP64, or
                                    EXA_PREC_FP32: an FP32 phase on FP32 staging arrays, then
-                                   FP64 correction sweeps; orders >= 5; the only form of
-                                   orders 8 and 9)                                          */
+                                   FP64 correction sweeps; orders >= 5; the default of
+                                   order 9)                                                 */
 
 int exa_aderdg_create(const exa_aderdg_config* cfg, exa_solver** out);
 
