@@ -947,17 +947,19 @@ __global__ __launch_bounds__(Ord<N>::NT) __attribute__((amdgpu_waves_per_eu(WPE,
 // one slice instead of N+1 and reads no array -- sum_t F0[t] iK1[l][t] = 1 (a
 // constant solution) and sum_t w[t] iK1[l][t] = xi[l] (one that grows like
 // time), so the new iterate is u + xi[l] L(u).  N = 9, 18^3 cells, 3.1 sweeps:
-// 6.72 -> 5.74 ms in FP64, 6.26 -> 5.33 mixed.  Bound by the traffic of the
+// 6.72 -> 5.74 ms in FP64, 6.26 -> 5.31 mixed.  Bound by the traffic of the
 // two arrays, which miss the L2.
 //
 // MIX: mixed precision (EXA_PREC_FP32).  The same sweep first runs on FP32
 // copies -- iterate and rhs as FP32 arrays in the first half of the slot,
 // flux slice and pencil constants as FP32 in the LDS, FP32 tables -- until
 // the residual reaches the FP32 rounding floor of the cell (or 2(N+1)
-// sweeps); the iterate is then widened into the slot's second array and at
-// most fp64_sweeps FP64 sweeps follow (stopping early on the FP64
+// sweeps); at most fp64_sweeps FP64 sweeps follow (stopping early on the FP64
 // criterion), from which the averages, extrapolation and volume integral
-// come, as in k_predictor's mixed form.
+// come, as in k_predictor's mixed form.  The first of them reads the FP32
+// iterate as it is, and one known to be the last stores only the time average
+// of its result: 5.31 -> 4.72 ms (N = 9, 18^3 cells) against a widened copy
+// and a result written and read again.
 template <int N, bool DEBUG, bool SRC = false, bool MIX = false>
 __global__ __launch_bounds__(Ord<N>::NT) void k_predictor_staged(
     const double* __restrict__ luh, double* __restrict__ lduh, double* __restrict__ qf, double* __restrict__ ff,
@@ -1007,6 +1009,11 @@ __global__ __launch_bounds__(Ord<N>::NT) void k_predictor_staged(
     double* q = slot;
     double* r = slot + SQ;
     int it = 0;
+    // the FP32 iterate, in the slot's first half: the input of the first FP64
+    // sweep, which writes into the second
+    const float* low = nullptr;
+    bool lowin = MIX;
+    auto input = [&](int i) { return MIX && lowin ? (double)low[i] : q[i]; };
     if constexpr (MIX) {
       // ---- FP32 phase ----
       float* qL = reinterpret_cast<float*>(slot);
@@ -1134,20 +1141,7 @@ __global__ __launch_bounds__(Ord<N>::NT) void k_predictor_staged(
           rL = tmp;
         }
       }
-      // the FP32 iterate (rL, in the slot's first half) widened into the
-      // second FP64 array, which becomes the input of the first FP64 sweep;
-      // every word is read and written by its own node's thread
-#pragma unroll 1
-      for (int t = 0; t < B; ++t) {
-        asm volatile("" : "+s"(tz));
-        const int sl = s + tz;
-        if (act)
-#pragma unroll
-          for (int v = 0; v < V; ++v) r[(t * V + v) * B3 + sl] = (double)rL[(t * V + v) * B3 + sl];
-      }
-      double* tmp = q;
-      q = r;
-      r = tmp;
+      low = rL;
       __syncthreads();  // the flux slice is free again
     }
     const int max64 = MIX ? it + fp64_sweeps : MaxIterations;
@@ -1155,6 +1149,8 @@ __global__ __launch_bounds__(Ord<N>::NT) void k_predictor_staged(
     while (!done) {
       ++it;
       const bool first = !MIX && it == 1;
+      // known to be the last sweep: of its result only the time average is kept
+      const bool last = MIX && !DEBUG && it == max64;
       double L[V];
 #pragma unroll 1
       for (int t = 0; t < (first ? 1 : B); ++t) {
@@ -1166,7 +1162,7 @@ __global__ __launch_bounds__(Ord<N>::NT) void k_predictor_staged(
           for (int v = 0; v < V; ++v) Q[v] = u[v];
           if (!first)
 #pragma unroll
-            for (int v = 0; v < V; ++v) Q[v] = q[(t * V + v) * B3 + sl];
+            for (int v = 0; v < V; ++v) Q[v] = input((t * V + v) * B3 + sl);
           EulerPDE::flux<double>(Q, F, gamma);
 #pragma unroll
           for (int v = 0; v < V; ++v) {
@@ -1243,18 +1239,21 @@ __global__ __launch_bounds__(Ord<N>::NT) void k_predictor_staged(
         double ri[B];
 #pragma unroll
         for (int t = 0; t < B; ++t) ri[t] = r[(t * V + v) * B3 + sv];
+        double mean = 0.0;
 #pragma unroll
         for (int t2 = 0; t2 < B; ++t2) {
           asm volatile("" : "+s"(tz));
           double acc = 0.0;
 #pragma unroll
           for (int t = 0; t < B; ++t) acc += ri[t] * c_tab[N + tz].iK1[t2][t];
-          const double dd = q[(t2 * V + v) * B3 + sv] - acc;
+          const double dd = input((t2 * V + v) * B3 + sv) - acc;
+          if (MIX) mean += acc * c_tab[N + tz].w[t2];
           if (act) {
             res += dd * dd;
-            r[(t2 * V + v) * B3 + sv] = acc;
+            if (!last) r[(t2 * V + v) * B3 + sv] = acc;
           }
         }
+        if (last && act) r[v * B3 + sv] = mean;
       }
       res = block_sum(res, red);
       __syncthreads();  // every thread has read red before the flux slice reuses it
@@ -1265,6 +1264,7 @@ __global__ __launch_bounds__(Ord<N>::NT) void k_predictor_staged(
         double* tmp = q;
         q = r;
         r = tmp;
+        lowin = false;
       } else if (first && act) {  // the input iterate, for its fluxes
 #pragma unroll 1
         for (int t = 0; t < B; ++t)
@@ -1287,7 +1287,7 @@ __global__ __launch_bounds__(Ord<N>::NT) void k_predictor_staged(
       if (act) {
         double Q[V], F[3][V];
 #pragma unroll
-        for (int v = 0; v < V; ++v) Q[v] = q[(t * V + v) * B3 + sl];
+        for (int v = 0; v < V; ++v) Q[v] = input((t * V + v) * B3 + sl);
         EulerPDE::flux<double>(Q, F, gamma);
         const double wt = T.w[t];
 #pragma unroll
@@ -1311,11 +1311,15 @@ __global__ __launch_bounds__(Ord<N>::NT) void k_predictor_staged(
 #pragma unroll 1
       for (int v = 0; v < V; ++v) {
         double a = 0.0;
+        if (MIX && !DEBUG && it == max64) {
+          a = r[v * B3 + s];
+        } else {
 #pragma unroll
-        for (int t = 0; t < B; ++t) {
-          const double qt = r[(t * V + v) * B3 + s];
-          a += qt * T.w[t];
-          if (DEBUG) dbg.lQi[(s * B + t) * V + v] = qt;
+          for (int t = 0; t < B; ++t) {
+            const double qt = r[(t * V + v) * B3 + s];
+            a += qt * T.w[t];
+            if (DEBUG) dbg.lQi[(s * B + t) * V + v] = qt;
+          }
         }
         sQh[v * B3 + s] = a;
         if (DEBUG) dbg.lQhi[s * V + v] = a;

@@ -51,6 +51,28 @@ def test_staged_first_sweep_vs_oracle(N, gravity):
             assert rel(g[k], o[k]) <= TOL, k
 
 
+@pytest.mark.parametrize("sweeps", [1, 2, 3])
+@pytest.mark.parametrize("N", [5, 8, 9])
+def test_staged_mixed_outputs_match_the_debug_form(N, sweeps):
+    """The staged mixed form keeps only the time average of a sweep known to be
+    its last; the per-cell outputs keep the whole iterate.  Same sums in the
+    same order: a few roundings (of fused products) apart, also where a
+    uniform cell stops before the last sweep."""
+    import exahype_amd as E
+    B2, B3 = (N + 1) ** 2, (N + 1) ** 3
+    s = E.ADERDGSolver(N, precision=E.PREC_FP32, contraction=E.CONTRACT_STAGED, fp64_sweeps=sweeps)
+    dx = np.array([1 / 27, 1 / 9, 1 / 20])
+    for seed in (1, None):
+        luh = _state(N, seed)
+        dt = 0.9 * O.stable_time_step_size(O.cfg(N), luh, dx)
+        g = s.spaceTimePredictor(luh, dx, dt)
+        o = (np.zeros(6 * B2 * 5), np.zeros(6 * B2 * 5), np.zeros(B3 * 5))
+        s.batch_prediction(*o, luh, dx, dt)
+        s.batch_flush()
+        assert rel(o[0], g["lQhbnd"]) <= 1e-14 * (N + 1)
+        assert rel(o[1], g["lFhbnd"]) <= 1e-14 * (N + 1)
+
+
 @pytest.mark.parametrize("N", range(1, 9))
 def test_deferred_predictions_vs_oracle(N):
     import exahype_amd as E
