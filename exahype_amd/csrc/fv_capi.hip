@@ -426,6 +426,7 @@ extern "C" int exa_fv_grid_create(exa_fv_solver* s, int nx, int ny, int nz, cons
   if (e == hipSuccess) e = hipMemcpy(g->state.p, st.data(), sizeof(double) * st.size(), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemset(g->cur.p, 0, sizeof(double) * psz * g->np);
   if (e == hipSuccess) e = hipMemset(g->nxt.p, 0, sizeof(double) * psz * g->np);
+  if (e == hipSuccess) e = hipStreamSynchronize(nullptr);  // the grid's stream does not wait for the null stream
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking);
   if (e != hipSuccess) {
     exa_set_error("fv grid setup: %s", hipGetErrorString(e));

@@ -64,3 +64,34 @@ def test_adaptive_grid_and_ensemble():
         o = E.Grid(E.ADERDGSolver(n), 4, 5, 3)
         o.set_initial_conditions(ic)
         assert np.array_equal(e.download(i), o.download())
+
+
+@pytest.mark.parametrize("dim,P,n", [(2, 10, (60, 50, 1)), (3, 11, (12, 11, 10))])
+def test_upload_right_after_creation_of_a_patch_grid(dim, P, n):
+    """A new grid's clearing is over when the grid is handed out: what is
+    written first on its own stream stays, and a step from it finds the ghost
+    layers of the other buffer cleared."""
+    import exahype_amd as E
+    s = E.FiniteVolumesSolver(dim, P, scheme=E.FV_GODUNOV if dim == 2 else E.FV_MUSCLHANCOCK)
+    rng = np.random.default_rng(P)
+    a = np.tile(np.array((1.0, 0.1, -0.2, 0.0 if dim == 2 else 0.3, 2.5)), int(np.prod(n)) * s.patch_size // 5)
+    a *= 1 + 0.01 * rng.random(a.size)
+    first = None
+    for _ in range(4):
+        g = E.FVGrid(s, *n)
+        g.upload(a)
+        assert np.array_equal(g.download(), a)
+        g.compute_dt()
+        g.step(1)
+        b = g.download()
+        first = b if first is None else first
+        assert np.array_equal(b, first)
+        ic = E.make_ic(5, xc=(0.4, 0.5, 0.6), L=0.05, amp=0.3, rho_inf=1.0, p_inf=1.0, uinf=(0.4, -0.3, 0.2))
+        h = E.FVGrid(s, *n)
+        h.set_initial_conditions(ic)
+        h = h.download()
+        g.set_initial_conditions(ic)  # cleared long ago
+        side, gh = s.side, (s.side - P) // 2
+        inner = (slice(None),) + (slice(gh, -gh),) * dim
+        shape = (int(np.prod(n)),) + (side,) * dim + (5,)
+        assert np.array_equal(h.reshape(shape)[inner], g.download().reshape(shape)[inner])
