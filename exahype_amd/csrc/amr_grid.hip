@@ -773,7 +773,6 @@ extern "C" int exa_amr_grid_create(exa_solver* s, const exa_amr_config* cfg, exa
   EXA_TRY(g->iters.ensure(sizeof(int) * nc));
   EXA_TRY(g->iter_sum.ensure(EXA_SWEEP_BYTES));
   EXA_CHECK(hipMemset(g->iter_sum.p, 0, EXA_SWEEP_BYTES));
-  EXA_CHECK(hipStreamSynchronize(nullptr));  // the grid's stream does not wait for the null stream
   EXA_TRY(up(g->face_kind, face_kind.data(), sizeof(int) * nc * 6));
   EXA_TRY(up(g->face_ref, face_ref.data(), sizeof(int) * nc * 6));
   EXA_TRY(up(g->anc_kids, anc_kids.data(), sizeof(int) * anc_kids.size()));
@@ -801,6 +800,7 @@ extern "C" int exa_amr_grid_create(exa_solver* s, const exa_amr_config* cfg, exa
   EXA_CHECK(hipMemset(g->cnt.p, 0, sizeof(unsigned long long) * NCNT));
   EXA_CHECK(hipMemset(g->status.p, 0, sizeof(int) * nc));
   EXA_CHECK(hipMemset(g->slot_of.p, 0xff, sizeof(int) * nc));
+  EXA_CHECK(hipStreamSynchronize(nullptr));  // the grid's stream does not wait for the null stream
   EXA_TRY(exa_amr_tables_dev(g->device, g->N, &g->amr_tab));
   EXA_TRY(exa_lim_tables_dev(g->device, g->N, &g->lim_tab));
   // LDS limits of the list kernels

@@ -11,7 +11,8 @@ CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
 
 
 @pytest.mark.parametrize("source,function", [("capi.hip", "exa_grid_create"), ("capi.hip", "exa_ensemble_create"),
-                                             ("fv_capi.hip", "exa_fv_grid_create")])
+                                             ("fv_capi.hip", "exa_fv_grid_create"),
+                                             ("amr_grid.hip", "exa_amr_grid_create")])
 def test_creation_waits_for_its_clearing(source, function):
     with open(os.path.join(CSRC, source)) as f:
         text = f.read()

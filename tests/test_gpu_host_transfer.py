@@ -95,3 +95,29 @@ def test_upload_right_after_creation_of_a_patch_grid(dim, P, n):
         inner = (slice(None),) + (slice(gh, -gh),) * dim
         shape = (int(np.prod(n)),) + (side,) * dim + (5,)
         assert np.array_equal(h.reshape(shape)[inner], g.download().reshape(shape)[inner])
+
+
+def test_upload_right_after_creation_of_an_adaptive_grid():
+    """The clearing of the statuses and patch slots is over when the grid is
+    handed out: the limiter's start, which the upload runs, is what a later
+    upload of the same state finds."""
+    import exahype_amd as E
+    s = E.ADERDGSolver(3)
+    cfg = E.amr_config(9, 3, (0.5, 0.5, 0.5), 0.25, (0.1, 0.05))
+    g = E.AMRGrid(s, cfg)
+    a = np.tile(np.array((1.0, 0.1, -0.2, 0.3, 2.5)), g.ncells * 64)
+    a *= 1 + 0.01 * np.random.default_rng(0).random(a.size)
+    level = g.cells()[:, 0]
+    a.reshape(-1, 64, 5)[np.flatnonzero(level == level.max())[::997], 5, 0] = -0.1  # troubled cells
+    del g
+    for _ in range(4):
+        g = E.AMRGrid(s, cfg)
+        g.upload(a)
+        first = g.limiter_status(), g.patches()
+        E.device_synchronize()
+        g.upload(a)
+        again = g.limiter_status(), g.patches()
+        assert np.array_equal(first[0], again[0]) and len(set(first[0])) > 1
+        for p in (first, again):
+            assert len(set(p[1][0])) == len(p[1][0]) and np.all(p[0][p[1][0]] != 0)
+        assert set(first[1][0]) == set(again[1][0])
