@@ -118,6 +118,7 @@ bool HostStage::ensure(size_t n) {
 int exa_transfer_nodes(HostStage& st, hipStream_t stream, double* blocks, double* user, long long units, int nodes,
                        bool up) try {
   if (units <= 0) return EXA_OK;
+  std::lock_guard<std::mutex> lk(st.mu);
   const size_t per = (size_t)V * nodes;
   const long long chunk = std::min(units, std::max<long long>(1, (long long)(CHUNK / (per * sizeof(double)))));
   if (!st.ensure(chunk * per)) return plain(stream, blocks, user, units, nodes, up);

@@ -2,6 +2,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <mutex>
+
 #include "common.h"
 
 #define EXA_ARG(cond, msg)                        \
@@ -66,7 +68,10 @@ struct DevBuf {
 
 // Two pinned buffers and their events, kept by the object whose solution they
 // move (at most 8 MB each, or one cell block), allocated by its first transfer.
+// One transfer at a time: host threads that move parts of one object take
+// their turns (the members of an ensemble share its buffers).
 struct HostStage {
+  std::mutex mu;  // held by exa_transfer_nodes
   double* buf[2] = {nullptr, nullptr};
   hipEvent_t ev[2] = {nullptr, nullptr};
   size_t words = 0;  // of each buffer

@@ -1,6 +1,8 @@
 """Uploads and downloads through the pinned buffers: every value at its place,
 bit for bit, for one short chunk, many chunks with a short last one, single
 cells larger than usual, special values, and a transfer behind queued steps."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -121,3 +123,42 @@ def test_upload_right_after_creation_of_an_adaptive_grid():
         for p in (first, again):
             assert len(set(p[1][0])) == len(p[1][0]) and np.all(p[0][p[1][0]] != 0)
         assert set(first[1][0]) == set(again[1][0])
+
+
+def _at_once(calls, rounds):
+    """Runs the calls in a host thread each, over and over; what they returned."""
+    got, gate = [[] for _ in calls], threading.Barrier(len(calls))
+
+    def work(i):
+        for _ in range(rounds):
+            gate.wait(60)
+            got[i].append(calls[i]())
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(calls))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    return got
+
+
+def test_downloads_of_one_handle_at_once():
+    """Host threads that read one object at the same time (the call releases
+    the interpreter's lock): members of an ensemble whose buffers differ in
+    size, and one grid, of several chunks each."""
+    import exahype_amd as E
+    ic = E.make_ic(5, xc=(0.4, 0.5, 0.6), L=0.05, amp=0.3, rho_inf=1.0, p_inf=1.0, uinf=(0.4, -0.3, 0.2))
+    members = [dict(order=n, cells=c) for n, c in ((3, (9, 9, 9)), (5, (14, 13, 12)), (7, (9, 10, 11)), (5, (13, 14, 11)))]
+    e = E.Ensemble(members)
+    e.set_initial_conditions([ic] * 4)
+    serial = [E.Ensemble([m]) for m in members]
+    for s in serial:
+        s.set_initial_conditions([ic])
+    want = [s.download(0) for s in serial]
+    # the ensemble's first transfers: its buffers grow while the others wait
+    for got, w in zip(_at_once([lambda i=i: e.download(i) for i in range(4)], 6), want):
+        assert all(np.array_equal(g, w) for g in got)
+    g = E.Grid(E.ADERDGSolver(5), 14, 13, 12)
+    g.set_initial_conditions(ic)
+    for got in _at_once([g.download] * 3, 4):
+        assert all(np.array_equal(x, want[1]) for x in got)
