@@ -12,8 +12,11 @@
 // patches of 15^3 volumes (295 MB) 90 ms; now 5 and 7 ms.
 #include <algorithm>
 #include <atomic>
+#include <chrono>
+#include <condition_variable>
 #include <cstring>
 #include <exception>
+#include <mutex>
 #include <thread>
 #include <vector>
 
@@ -24,6 +27,10 @@ constexpr int V = 5;
 constexpr size_t CHUNK = 8u << 20;         // bytes of one buffer
 constexpr size_t PER_THREAD = 2u << 20;    // a thread more for so many bytes
 constexpr int MAX_THREADS = 8;
+// A helper polls for its next chunk so long and then sleeps: more than a chunk
+// takes on the link (150 us), far less than the steps that a transfer may have
+// to wait for.
+constexpr std::chrono::microseconds POLL{500};
 
 // words of whole units; UP: reference layout to blocks
 template <bool UP>
@@ -70,17 +77,47 @@ int plain(hipStream_t stream, double* blocks, double* user, long long units, int
 }
 
 // What the threads that share the copying of every chunk know.
-struct Progress {
-  std::atomic<long long> open{0};    // chunks that may be copied
+class Progress {
+  std::atomic<long long> open_{0};  // chunks that may be copied
+  std::atomic<bool> stop_{false};
+  std::mutex mu_;  // of the changes, for those that sleep
+  std::condition_variable changed_;
+
+ public:
   std::atomic<long long> copied{0};  // parts copied by the helpers
   std::atomic<int> parts{1};         // of a chunk; set before the first one opens
-  std::atomic<bool> stop{false};
+  void open(long long chunks) {
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      open_.store(chunks, std::memory_order_release);
+    }
+    changed_.notify_all();
+  }
+  void stop() {
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      stop_.store(true, std::memory_order_release);
+    }
+    changed_.notify_all();
+  }
+  // Waits until chunk k may be copied; false: it will not be.
+  bool wait(long long k) {
+    auto open = [&] { return open_.load(std::memory_order_acquire) > k; };
+    auto stopped = [&] { return stop_.load(std::memory_order_acquire); };
+    const auto until = std::chrono::steady_clock::now() + POLL;
+    while (!open() && !stopped() && std::chrono::steady_clock::now() < until) std::this_thread::yield();
+    if (!open() && !stopped()) {
+      std::unique_lock<std::mutex> lk(mu_);
+      changed_.wait(lk, [&] { return open() || stopped(); });
+    }
+    return open();
+  }
 };
 struct Helpers {
   Progress& progress;
   std::vector<std::thread> threads;
   ~Helpers() {
-    progress.stop.store(true, std::memory_order_release);
+    progress.stop();
     for (auto& t : threads) t.join();
   }
 };
@@ -138,10 +175,7 @@ int exa_transfer_nodes(HostStage& st, hipStream_t stream, double* blocks, double
   };
   auto help = [&](int part) {
     for (long long k = 0; k < nchunks; ++k) {
-      while (pr.open.load(std::memory_order_acquire) <= k) {
-        if (pr.stop.load(std::memory_order_acquire)) return;
-        std::this_thread::yield();
-      }
+      if (!pr.wait(k)) return;
       copy(k, part, pr.parts.load(std::memory_order_relaxed));
       pr.copied.fetch_add(1, std::memory_order_release);
     }
@@ -166,7 +200,7 @@ int exa_transfer_nodes(HostStage& st, hipStream_t stream, double* blocks, double
     return EXA_OK;
   };
   auto share = [&](long long k) {  // copies chunk k with the helpers
-    pr.open.store(k + 1, std::memory_order_release);
+    pr.open(k + 1);
     copy(k, 0, nparts);
     while (pr.copied.load(std::memory_order_acquire) < (k + 1) * (nparts - 1)) std::this_thread::yield();
   };

@@ -162,3 +162,29 @@ def test_downloads_of_one_handle_at_once():
     g.set_initial_conditions(ic)
     for got in _at_once([g.download] * 3, 4):
         assert all(np.array_equal(x, want[1]) for x in got)
+
+
+@pytest.mark.parametrize("up", [False, True])
+def test_transfer_behind_steps_leaves_the_cores_idle(up):
+    """A transfer that has to wait for queued steps sleeps meanwhile: the
+    process may use the calling thread's core and one more, not one per thread
+    that will share the copying."""
+    import time
+    import exahype_amd as E
+    g = E.Grid(E.ADERDGSolver(5), 27, 27, 27)
+    ic = E.make_ic(5, xc=(0.4, 0.5, 0.6), L=0.05, amp=0.3, rho_inf=1.0, p_inf=1.0, uinf=(0.4, -0.3, 0.2))
+    g.set_initial_conditions(ic)
+    a = g.download()
+    g.compute_dt()
+    g.use_graph(True)
+    g.step(2)
+    g.sync()
+    g.step(500)
+    t, c = time.perf_counter(), time.process_time()
+    if up:
+        g.upload(a)
+    else:
+        a = g.download()
+    t, c = time.perf_counter() - t, time.process_time() - c
+    assert t > 0.2  # it waited
+    assert c < 2.5 * t
