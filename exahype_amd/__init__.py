@@ -733,7 +733,7 @@ class FVGrid:
 
     def kernel_times(self):
         """(ms summed, launches) per phase since the last call: ghost layers,
-        MUSCL-Hancock states, update, time step."""
+        (unused), update with the new states' CFL bounds, time step from them."""
         t = np.zeros(4)
         c = (C.c_longlong * 4)()
         _check(_lib.exa_fv_grid_kernel_times(self._h, _p(t), c))

@@ -240,7 +240,8 @@ struct exa_fv_grid {
   exa_bc bc{};
   hipStream_t stream = nullptr;
   bool dt_valid = false;  // a stable dt has been computed (sync checks it from then on)
-  // per-phase kernel timing (0 ghost layers, 1 unused, 2 update, 3 dt)
+  // per-phase kernel timing (0 ghost layers, 1 unused, 2 update with the new
+  // states' CFL bounds, 3 time step out of the update's minima)
   bool timing = false;
   std::vector<std::vector<hipEvent_t>> marks;  // 5 events per timed step
   double times[4] = {0, 0, 0, 0};
@@ -581,10 +582,10 @@ extern "C" int exa_fv_grid_step(exa_fv_grid* g, int nsteps) {
                              g->slots(1), g->dx, g->dt_cur()));
     if (m[3]) EXA_CHECK(hipEventRecord(m[3], g->stream));
     g->cur.swap(g->nxt);
-    if (m[4]) EXA_CHECK(hipEventRecord(m[4], g->stream));  // the update's part of the time step included above
     hipLaunchKernelGGL(k_fv_dt_advance, dim3(1), dim3(64), 0, g->stream, g->dt_cur(), g->adm(), g->time(),
                        g->slots(0), g->slots(1));
     EXA_CHECK(hipGetLastError());
+    if (m[4]) EXA_CHECK(hipEventRecord(m[4], g->stream));
   }
   return EXA_OK;
 }
