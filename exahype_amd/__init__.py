@@ -130,6 +130,7 @@ EXPORTS = [
     "exa_ensemble_create", "exa_ensemble_destroy", "exa_ensemble_set_initial_conditions", "exa_ensemble_compute_dt",
     "exa_ensemble_use_graph", "exa_ensemble_step", "exa_ensemble_sync", "exa_ensemble_download",
     "exa_ensemble_total_picard_iterations", "exa_autotune",
+    "exa_autotune_recorded",
     "exa_grid_limiter_snapshot", "exa_grid_limiter_check", "exa_grid_limiter_project",
 ]
 
@@ -219,6 +220,7 @@ def load_library(path=LIB_PATH):
     L.exa_device_copy.argtypes = [C.c_void_p, C.c_void_p, LL, P(C.c_float)]
     L.exa_selftest_mfma.argtypes = [I, C.c_void_p, C.c_void_p, C.c_void_p]
     L.exa_autotune.argtypes = [I, I, I, P(I), P(I), _D]
+    L.exa_autotune_recorded.argtypes = [I, I, P(I), P(I)]
     L.exa_grid_limiter_snapshot.argtypes = [C.c_void_p, I]
     L.exa_grid_limiter_check.argtypes = [C.c_void_p, C.c_double, C.c_double, P(LL), P(I)]
     L.exa_grid_limiter_project.argtypes = [C.c_void_p, I, C.c_void_p, LL, P(I)]
@@ -1164,10 +1166,21 @@ class Ensemble:
 
 def autotune(order, precision=PREC_FP64, ncells=32):
     """Times the predictor variants of one order/precision on this device and
-    records the fastest; returns (waves_per_simd, contraction, times_ms)."""
+    records the fastest if it beats the untuned default (autotune_recorded);
+    returns the fastest as (waves_per_simd, contraction, times_ms)."""
     L = load_library()
     _check(L.exa_init(0))
     w, c = C.c_int(0), C.c_int(0)
     ms = np.zeros(6)
     _check(L.exa_autotune(order, precision, ncells, C.byref(w), C.byref(c), _p(ms)))
     return w.value, c.value, ms
+
+
+def autotune_recorded(order, precision=PREC_FP64):
+    """(waves_per_simd, contraction) that solvers left at the defaults take;
+    (0, 0): nothing is recorded and the untuned default serves."""
+    L = load_library()
+    _check(L.exa_init(0))
+    w, c = C.c_int(0), C.c_int(0)
+    _check(L.exa_autotune_recorded(order, precision, C.byref(w), C.byref(c)))
+    return w.value, c.value

@@ -265,6 +265,15 @@ struct TunedVariant {
   int contraction = 0;
 };
 static TunedVariant g_tuned[64][EXA_MAX_ORDER + 1][4];
+// Contraction of the solver that exa_autotune measures the others against:
+// EXA_CONTRACT_DEFAULT without what has been recorded.
+static constexpr int CONTRACT_UNTUNED = -1;
+static TunedVariant tuned(const exa_aderdg_config& c, int dev) {
+  return c.contraction == CONTRACT_UNTUNED ? TunedVariant{} : g_tuned[dev & 63][c.order][c.precision & 3];
+}
+static bool untuned_default(const exa_aderdg_config& c, int dev) {
+  return c.contraction <= EXA_CONTRACT_DEFAULT && tuned(c, dev).contraction == 0;
+}
 
 // The staged predictor: orders 8, 9, chosen explicitly, or at N = 7 in FP64
 // where predictor_history does not serve (the gravity source, per-cell
@@ -273,8 +282,7 @@ static TunedVariant g_tuned[64][EXA_MAX_ORDER + 1][4];
 static bool predictor_staged(const exa_aderdg_config& c, int dev) {
   if (exa_pde_generic(c.pde)) return false;
   if (c.order >= 8 || c.contraction == EXA_CONTRACT_STAGED) return true;
-  return c.order == 7 && c.precision == EXA_PREC_FP64 && c.contraction == EXA_CONTRACT_DEFAULT &&
-         g_tuned[dev & 63][7][EXA_PREC_FP64].contraction == 0;  // exa_autotune's choice wins
+  return c.order == 7 && c.precision == EXA_PREC_FP64 && untuned_default(c, dev);  // exa_autotune's choice wins
 }
 
 // The default predictor of the Euler equations in FP64 or with FP32 sweeps
@@ -285,8 +293,8 @@ static bool predictor_staged(const exa_aderdg_config& c, int dev) {
 static bool predictor_history(const exa_aderdg_config& c, int dev) {
   return c.pde == EXA_PDE_EULER && !c.linear && c.order >= EXA_HISTORY_MIN_ORDER &&
          c.order <= EXA_HISTORY_MAX_ORDER &&
-         (c.precision == EXA_PREC_FP64 || c.precision == EXA_PREC_FP32) && c.contraction == EXA_CONTRACT_DEFAULT &&
-         c.waves_per_simd == 0 && g_tuned[dev & 63][c.order][c.precision].contraction == 0;
+         (c.precision == EXA_PREC_FP64 || c.precision == EXA_PREC_FP32) && c.waves_per_simd == 0 &&
+         untuned_default(c, dev);
 }
 
 // Launch extras of a single-grid predictor launch: the gravity source of
@@ -315,7 +323,7 @@ static int predictor_form(const exa_aderdg_config& c, int N, int dev) {
     case EXA_CONTRACT_PENCIL_PAIR: return exa::FORM_PENCIL_PAIR;
     default: break;
   }
-  const int tc = g_tuned[dev & 63][N][c.precision & 3].contraction;
+  const int tc = tuned(c, dev).contraction;
   if (tc) return tc == EXA_CONTRACT_NODE ? exa::FORM_NODE
                                          : (tc == EXA_CONTRACT_PENCIL_PAIR ? exa::FORM_PENCIL_PAIR : exa::FORM_PENCIL);
   // measured at 81^3 cells, FP64 predictor ms (pencil / node / pencil pairs):
@@ -327,7 +335,7 @@ extern "C" int exa_aderdg_create(const exa_aderdg_config* cfg, exa_solver** out)
   EXA_ARG(cfg && out, "null pointer");
   EXA_ARG(cfg->order >= 1 && cfg->order <= 9, "order must be 1..9");
   EXA_ARG(cfg->order <= 7 || cfg->precision <= EXA_PREC_FP32,
-          "orders 8 and 9 run the staged predictor: FP64 or FP32 sweeps with FP64 correction");
+          "orders 8 and 9 have FP64 or FP32 sweeps with FP64 correction");
   EXA_ARG(cfg->contraction != EXA_CONTRACT_STAGED ||
               (cfg->precision <= EXA_PREC_FP32 && cfg->order >= EXA_STAGED_MIN_ORDER),
           "the staged predictor is FP64 or FP32 + FP64 and built for orders 5..9");
@@ -1411,7 +1419,7 @@ extern "C" int exa_grid_fused_reruns(exa_grid* g, long long* reruns) {
 // (two waves per SIMD trade a few spilled registers for latency hiding).
 static int predictor_waves_per_simd(const exa_aderdg_config& c, int N, int dev) {
   if (c.waves_per_simd == 1 || c.waves_per_simd == 2) return c.waves_per_simd;
-  const int tw = g_tuned[dev & 63][N][c.precision & 3].wpe;
+  const int tw = tuned(c, dev).wpe;
   if (tw) return tw;
   // measured at 81^3 cells: two waves per SIMD is 1.6x faster at N=5
   return N <= 5 ? 2 : 1;
@@ -2027,7 +2035,7 @@ extern "C" int exa_ensemble_total_picard_iterations(exa_ensemble* e, long long* 
 // ---------------------------------------------------------------------------
 // Autotuner of the predictor's launch variant: times every (waves per SIMD,
 // contraction form) pair of one order and precision on a synthetic vortex
-// grid and records the fastest for this device.
+// grid and records the fastest for this device, if it beats the default.
 extern "C" int exa_autotune(int order, int precision, int ncells, int* waves_per_simd, int* contraction,
                             double ms[6]) {
   EXA_ARG(order >= 1 && order <= 7, "order must be 1..7");
@@ -2058,6 +2066,7 @@ extern "C" int exa_autotune(int order, int precision, int ncells, int* waves_per
     exa_solver* s = nullptr;
     exa_grid* g = nullptr;
     EXA_TRY(exa_aderdg_create(&cfg, &s));
+    if (cform == EXA_CONTRACT_DEFAULT) s->cfg.contraction = CONTRACT_UNTUNED;
     int r = exa_grid_create(s, ncells, ncells, ncells, nullptr, nullptr, &g);
     *t = 1e300;
     if (r == EXA_OK) r = exa_grid_set_initial_conditions(g, &ic);
@@ -2091,13 +2100,20 @@ extern "C" int exa_autotune(int order, int precision, int ncells, int* waves_per
     }
   // solvers left at the defaults take the fastest of the six unless the
   // untuned default is faster still
-  g_tuned[dev & 63][order][precision] = TunedVariant{};
   EXA_TRY(variant(0, EXA_CONTRACT_DEFAULT, &deflt));
-  if (best < deflt) {
-    g_tuned[dev & 63][order][precision].wpe = bw;
-    g_tuned[dev & 63][order][precision].contraction = bc;
-  }
+  g_tuned[dev & 63][order][precision] = best < deflt ? TunedVariant{bw, bc} : TunedVariant{};
   if (waves_per_simd) *waves_per_simd = bw;
   if (contraction) *contraction = bc;
+  return EXA_OK;
+}
+
+extern "C" int exa_autotune_recorded(int order, int precision, int* waves_per_simd, int* contraction) {
+  EXA_ARG(order >= 1 && order <= EXA_MAX_ORDER, "order must be 1..9");
+  EXA_ARG(precision >= EXA_PREC_FP64 && precision <= EXA_PREC_BF16_MFMA, "precision");
+  int dev = 0;
+  EXA_CHECK(hipGetDevice(&dev));
+  const TunedVariant& t = g_tuned[dev & 63][order][precision];
+  if (waves_per_simd) *waves_per_simd = t.wpe;
+  if (contraction) *contraction = t.contraction;
   return EXA_OK;
 }

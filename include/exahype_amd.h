@@ -159,13 +159,16 @@ int exa_aderdg_create(const exa_aderdg_config* cfg, exa_solver** out);
 
 /* Autotuner: times the predictor of one order and precision in every launch
  * variant (1 or 2 waves per SIMD x EXA_CONTRACT_PENCIL, _NODE, _PENCIL_PAIR)
- * on an ncells^3 vortex grid and records the fastest for this device; solvers
- * created later with waves_per_simd = 0 and contraction = 0 use it unless the
- * untuned default was measured faster still.  Reports
- * the choice and the six average launch times (ms, waves-major: w1-pencil,
- * w1-node, w1-pair, w2-pencil, w2-node, w2-pair).  No counterpart in the
- * reference. */
+ * and in the untuned default on an ncells^3 vortex grid.  Records the fastest
+ * variant for this device if it beat the default, for solvers with
+ * waves_per_simd = 0 and contraction = 0; otherwise these keep the default and
+ * nothing is recorded (exa_autotune_recorded).  Reports the fastest of the six
+ * either way and their average launch times (ms, waves-major: w1-pencil,
+ * w1-node, w1-pair, w2-pencil, w2-node, w2-pair).  After an error an earlier
+ * record stands.  No counterpart in the reference. */
 int exa_autotune(int order, int precision, int ncells, int* waves_per_simd, int* contraction, double ms[6]);
+/* What is recorded for the current device; 0 and 0: the untuned default serves. */
+int exa_autotune_recorded(int order, int precision, int* waves_per_simd, int* contraction);
 int exa_aderdg_destroy(exa_solver* s);
 
 /* ADERDGSolver::spaceTimePredictor (E/solvers/ADERDGSolver.h:1049-1059;
