@@ -9,9 +9,10 @@
 // hence the resident waves -- and the number of slices decide.  Against the
 // other forms it takes one slice instead of B in the first sweep (HistTables
 // a, b), half the products of the spatial contraction (ev, od), no pencil
-// constants (the scale is applied once per node), and 180 instead of 254
-// registers at N = 5 (pin, park).  ms per launch (FP64 / FP32 sweeps, vortex
-// grid; before: the fastest of the other forms):
+// constants (the scale is applied once per node), and fewer registers (pin,
+// park): at N = 5 168 in FP64 and 158 with FP32 sweeps, three waves per SIMD,
+// instead of 255 and 239.  ms per launch (FP64 / FP32 sweeps, vortex grid;
+// before: the fastest of the other forms):
 //   N = 1  45^3   0.42 -> 0.23     0.45 -> 0.23
 //   N = 2  45^3   0.72 -> 0.48     0.68 -> 0.40
 //   N = 3  45^3   1.23 -> 0.81     1.07 -> 0.66
@@ -80,14 +81,22 @@ struct HistOrd {
   static constexpr int SLICE = 3 * V * Ord<N>::BLK + 32;
   // Time levels of a sweep's input iterate that wait in the LDS for the
   // residual and the flux averages: FP64 sweeps (doubles), and the one FP64
-  // sweep after FP32 sweeps (floats).  As many as the LDS holds beside the
-  // slices of the workgroups that the registers admit.
+  // sweep after FP32 sweeps (floats).  Never more than the LDS holds beside the
+  // slices of the workgroups that the registers admit; ms per launch with none
+  // / these / as many as that (meshes as above):
+  //           FP64                            FP32 sweeps
+  //   N = 4   1.81 / none / 1.86 (2)          1.52 / none / 1.52 (4)
+  //   N = 5   5.06 / 4.05 (2, the most)       3.93 / 3.47 (4) / 3.49 (5)
+  //   N = 6   2.25 / none / 2.46 (7)          2.35 / 1.93 (5, the most)
+  //   N = 7   3.36 / 3.34 (4, the most)       2.79 / 2.90 (8, the most)
+  //   N = 8   2.96 / 2.66 (2, the most)       1.66 / 1.45 (4) / 1.44 (5)
   static constexpr int PARK64 = N == 5 ? 2 : N == 7 ? 4 : N == 8 ? 2 : 0;
   static constexpr int PARKMX = N == 5 ? 4 : N == 6 ? 5 : N == 7 ? 8 : N == 8 ? 4 : 0;
   // Waves per SIMD.  N = 5, ms at 45^3 with 2 / 3 / 4: FP64 5.1 / 4.2 / 7.4
   // (spills), mixed 4.5 / 3.65 / 3.8.  N = 6 is six waves per workgroup, of
-  // which two fit only at 4 per SIMD: FP64 spills there (2.3 / - / 3.9 at
-  // 27^3), mixed does not (2.1 / 2.1 / 1.9).  N = 7: 3.4 / 4.7 and 2.9 / 3.5.
+  // which two fit only at 4 per SIMD: FP64 spills too much there (2.3 / - / 3.9
+  // at 27^3), mixed 164 bytes a lane (2.1 / 2.1 / 1.9).  N = 7: 3.4 / 4.7 and
+  // 2.9 / 3.5.
   // N = 3 (one wave per cell): 0.88 / 0.81 / 0.81 and 0.78 / 0.68 / 0.66.
   static constexpr int WPE64 = N <= 3 ? 4 : N == 6 || N == 7 ? 2 : 3;
   static constexpr int WPEMX = N == 7 ? 2 : N <= 3 || N == 6 ? 4 : 3;
@@ -98,22 +107,17 @@ struct HistOrd {
   }
 };
 
-// A zero the compiler cannot see through, available once `after` is computed:
-// a table or memory read indexed with it is issued there and not hoisted to
-// where its registers would be held for long.
-template <typename T>
-__device__ __forceinline__ int zero_after(T after) {
-  int z;
-  asm volatile("s_mov_b32 %0, 0" : "=s"(z) : "v"(after));
-  return z;
-}
 // Keeps a value where it is computed: without it the time contraction's sums,
 // not needed before the end of the sweep, sink there, and the terms of every
-// slice are held in their place (N = 5: 254 registers and spills for 188).
+// slice are held in their place (N = 5 in FP64, nothing parked, two waves per
+// SIMD: 243 registers for 190; with two levels parked 174).
 template <typename T>
 __device__ __forceinline__ void pin(T& x) {
   asm volatile("" : "+v"(x));
 }
+// A zero the compiler cannot see through: a table or memory read indexed with
+// it is issued there and not hoisted to where its registers would be held for
+// long.
 __device__ __forceinline__ int opaque_zero() {
   int z;
   asm volatile("s_mov_b32 %0, 0" : "=s"(z));
@@ -381,11 +385,13 @@ __device__ __forceinline__ int hist_sweeps(T (&q)[Ord<N>::B][V], T (&r)[Ord<N>::
 //   F  node owners evaluate the flux of q[t] and store it in the direction
 //      layouts;
 //   P  the 3 V B^2 pencils of the slice are contracted with Kxi in place;
-//   A  node owners keep the sum R[t] = w_t dt (Px/(w_x dx) + Py/(w_y dy) +
-//      Pz/(w_z dz)).
-// At the end of the sweep the node's history R becomes the next iterate in
-// place (hist_next).  The first sweep starts from data constant in time and
-// needs one slice (c_tt).
+//   A  node owners form R = w_t dt (Px/(w_x dx) + Py/(w_y dy) + Pz/(w_z dz))
+//      and take iK1[t'][t] R off every level t' of the next iterate qn, which
+//      starts from a[t'] u.
+// The input iterate q stays beside qn, partly in the LDS (park), for the
+// residual at the end of the sweep and the flux averages after the last one.
+// The first sweep starts from data constant in time and needs one slice
+// (tables a, b).
 // MIXED: FP32 sweeps to the FP32 rounding floor of the cell, then fp64_sweeps
 // FP64 sweeps.  ONE: fp64_sweeps is 1, so that sweep needs no residual and
 // its input iterate stays in FP32 and dies slice by slice.  USKIP: a cell

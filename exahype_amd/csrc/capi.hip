@@ -80,7 +80,7 @@ static PredFn predictor_kernel(bool debug, int prec, int wpe, int form, bool usk
     case 5: return exa_pred_kernel_5(debug, prec, wpe, form, uskip);
     case 6: return exa_pred_kernel_6(debug, prec, wpe, form, uskip);
     case 7: return exa_pred_kernel_7(debug, prec, wpe, form, uskip);
-    default: return nullptr;  // orders 8, 9: exa_pred_staged_kernel
+    default: return nullptr;  // not built for orders 8 and 9
   }
 }
 

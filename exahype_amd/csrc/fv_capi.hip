@@ -58,7 +58,7 @@ extern "C" int exa_fv_create(const exa_fv_config* cfg, exa_fv_solver** out) {
   EXA_ARG(cfg->scheme == EXA_FV_GODUNOV || (cfg->scheme == EXA_FV_MUSCLHANCOCK && cfg->dim == 3),
           "scheme: Godunov (2D/3D) or MUSCL-Hancock (3D)");
   EXA_ARG(cfg->scheme != EXA_FV_MUSCLHANCOCK || cfg->patch <= 15,
-          "MUSCL-Hancock patches up to 15^3 (the half-step terms of a patch are held in LDS)");
+          "MUSCL-Hancock patches up to 15^3 (the sizes that the kernel is built for)");
   EXA_ARG(cfg->nvar == 5 && cfg->npar == 0, "5 variables, no parameters");
   EXA_ARG((cfg->pde == EXA_PDE_EULER && cfg->dim == 3) || (cfg->pde == EXA_PDE_EULERFV2D && cfg->dim == 2),
           "pde: EXA_PDE_EULER in 3D, EXA_PDE_EULERFV2D in 2D");

@@ -3,12 +3,14 @@
 //
 // Device layout of a patch: structure of arrays over the patch including
 // its ghost layers, [patch][v][cell], cell = (k*S + j)*S + i (3D) or j*S + i
-// (2D), S = patch + 2*ghost.  Updates are written in gather form: one thread
+// (2D), S = patch + 2*ghost.  Godunov is written in gather form: one thread
 // per interior cell evaluates the Rusanov fluxes of its 2*DIM faces and
 // applies them in the reference's order (x-, x+, y-, y+, z-, z+), so each
 // cell's accumulation matches the reference's face loops
-// (kernels/finitevolumes/godunov/c/{2d,3d}/godunov.cpph,
-// kernels/finitevolumes/musclhancock/c/3d/musclhancock.cpph).
+// (kernels/finitevolumes/godunov/c/{2d,3d}/godunov.cpph).  MUSCL-Hancock
+// (kernels/finitevolumes/musclhancock/c/3d/musclhancock.cpph) forms every flux
+// once and adds up a cell's fluxes in another order, before its state: a few
+// roundings apart.
 #pragma once
 #include "common.h"
 #include "pde_euler.h"
@@ -209,7 +211,7 @@ __device__ inline double wave_uniform(double x) {
 // waves.  36 KB of LDS at 11^3 let four workgroups share a compute unit, and
 // cover each other's waits, if 168 registers hold a thread: values that wait
 // longest stay in the LDS or are loaded again, since a spilled register's
-// reload also waits for every load in flight (24 spills: 344 us).
+// reload also waits for every load in flight (24 spills: 344 us; 2 are left).
 // 12 x 13 x 14 patches of 11^3: 232 us, 258 with the new states' time step (a
 // pass of its own: 41).  Forming the states of each subcell
 // and face where they are used, every state four times: 527; one thread per
@@ -593,7 +595,7 @@ __global__ __launch_bounds__(256) void k_fv_ghosts(double* __restrict__ luh, con
 // (E/solvers/FiniteVolumesSolver.cpp:689-728): the mirrored layer of the
 // boundary-layer extraction through boundaryValues.  One workgroup per patch,
 // launched where an axis is closed; kept apart because the analytical boundary
-// values take 130 registers.
+// values take 157 registers in 2D and 168 in 3D (the copy alone 22 and 58).
 template <int DIM>
 __global__ __launch_bounds__(256) void k_fv_boundary(double* __restrict__ luh, const int* __restrict__ nbr,
                                                      PatchGeom g, int npatch, FvBoundary fb) {

@@ -67,7 +67,8 @@ struct DevBuf {
 };
 
 // Two pinned buffers and their events, kept by the object whose solution they
-// move (at most 8 MB each, or one cell block), allocated by its first transfer.
+// move (at most 8 MB each, or one cell block), allocated by its first transfer
+// and kept for the next ones: up to 16 MB of pinned memory an object.
 // One transfer at a time: host threads that move parts of one object take
 // their turns (the members of an ensemble share its buffers).
 struct HostStage {

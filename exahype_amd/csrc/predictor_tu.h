@@ -42,7 +42,8 @@ PredFn exa_pred_history_kernel(int order, bool mixed, int fp64_sweeps, bool uski
 int exa_pred_history_lds_bytes(int order, bool mixed, int fp64_sweeps, bool uskip = false);
 hipError_t exa_pred_history_init(const DGTables* tab, const DGTablesF* tabf);
 
-// Staged predictor (pred_staged.hip; orders 5..9, the only form of 8 and 9):
+// Staged predictor (pred_staged.hip; orders 5..9, the only form of 9, of order
+// 8 with the gravity source or per-cell outputs):
 // the space-time iterate lives in a staging slot of global memory per
 // workgroup (2 B^4 V doubles), the grid is persistent (one workgroup per
 // slot, cells strided by the grid size).
