@@ -44,6 +44,12 @@ def predictor_flops_per_cell(N, iters):
     return iters * (8 * NVAR * B ** 5 + B ** 4 * (PHI_FLUX + 5 * NVAR)) + 14 * NVAR * B ** 4 + 24 * NVAR * B ** 3
 
 
+def predictor_name(N, sweeps, default):
+    """The predictor kernel as the line and profiles/traffic.json name it;
+    default: no launch variant asked for, vector sweeps."""
+    return "k_predictor%s<%d, %s>" % ("_history" if default and N <= 8 else "", N, sweeps)
+
+
 def measured_traffic(kernel, n, N):
     """HBM bytes per launch of `kernel` from the counter runs summarised in
     profiles/traffic.json (FETCH_SIZE and WRITE_SIZE, each scaled by what the
@@ -312,9 +318,8 @@ def main():
         flops = f_lp + f64
         peak_lp = PEAK_BF16_TFLOPS if best["prec"] == E.PREC_BF16_MFMA else PEAK_FP32_TFLOPS
         peak = flops / (f_lp / peak_lp + f64 / PEAK_FP64_TFLOPS)
-        hist = best["prec"] == E.PREC_FP32 and args.contraction == 0 and args.waves_per_simd == 0 and N <= 8
-        kname = "k_predictor%s<%d, %s + %d FP64 sweep(s)>" % ("_history" if hist else "", N, best["name"],
-                                                              best["sweeps_fp64"])
+        default = best["prec"] == E.PREC_FP32 and args.contraction == 0 and args.waves_per_simd == 0
+        kname = predictor_name(N, "%s + %d FP64 sweep(s)" % (best["name"], best["sweeps_fp64"]), default)
         # what bounds each part: FP32 sweeps on the vector ALU (no packed
         # FP32), MFMA forms on the matrix cores, FP64 sweeps and tail on the
         # FP64 vector ALU
@@ -323,8 +328,7 @@ def main():
     else:
         flops = predictor_flops_per_cell(N, sweeps) * ncells
         peak = PEAK_FP64_TFLOPS
-        hist = args.contraction == 0 and args.waves_per_simd == 0 and N <= 8
-        kname = "k_predictor%s<%d, FP64>" % ("_history" if hist else "", N)
+        kname = predictor_name(N, "FP64", args.contraction == 0 and args.waves_per_simd == 0)
         bound = "fp64_valu"
     achieved = flops / (pred_ms * 1e-3) / 1e12
 
