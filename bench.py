@@ -39,7 +39,9 @@ NVAR = 5
 def predictor_flops_per_cell(N, iters):
     """Algorithmic FLOP of one predictor launch per cell: I Picard sweeps of
     8 V B^5 contraction flops + B^4 (flux + 5V), then time averages and the
-    volume integral (14 V B^4) and the face extrapolation (24 V B^3)."""
+    volume integral (14 V B^4) and the face extrapolation (24 V B^3).  The first
+    sweep counts in full, though its iterate is constant in time and the default
+    forms execute one slice of it."""
     B = N + 1
     return iters * (8 * NVAR * B ** 5 + B ** 4 * (PHI_FLUX + 5 * NVAR)) + 14 * NVAR * B ** 4 + 24 * NVAR * B ** 3
 

@@ -206,13 +206,13 @@ __device__ inline double wave_uniform(double x) {
 // The first ghost layer receives the patch-boundary face updates as in the
 // reference.  The planes above are loaded while a plane is worked on.
 //
-// Bound by vector FP64 and its latencies: about 1000 instructions a plane and
-// wave (15 divisions, 6 square roots), two barriers between at most five
-// waves.  36 KB of LDS at 11^3 let four workgroups share a compute unit, and
+// Bound by vector FP64 (the ALUs are busy for 77 % of a launch at 11^3): 1155
+// instructions a plane and wave (15 divisions, 6 square roots), two barriers
+// between at most five waves.  36 KB of LDS at 11^3 let four workgroups share a compute unit, and
 // cover each other's waits, if 168 registers hold a thread: values that wait
 // longest stay in the LDS or are loaded again, since a spilled register's
 // reload also waits for every load in flight (24 spills: 344 us; 2 are left).
-// 12 x 13 x 14 patches of 11^3: 232 us, 258 with the new states' time step (a
+// 12 x 13 x 14 patches of 11^3: 232 us, 254 with the new states' time step (a
 // pass of its own: 41).  Forming the states of each subcell
 // and face where they are used, every state four times: 527; one thread per
 // two subcells, a patch's states in the LDS at once, one workgroup per compute
